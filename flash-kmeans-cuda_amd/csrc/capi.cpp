@@ -216,7 +216,7 @@ struct LoopBuffers {
   int32_t* perm = nullptr;
   float* sums = nullptr;
   int32_t* counts = nullptr;
-  float* shift = nullptr;  // one slot per iteration
+  float* shift = nullptr;  // one slot per iteration (finalize not fused)
   int32_t* ctrl = nullptr; // [0] converged, [1] iterations run
   void* sort_ws = nullptr;
   size_t sort_ws_bytes = 0;
@@ -528,9 +528,18 @@ int lloyd_run(const void* x, const void* init, void* centroids,
   zf.n0 = 4;
   label_sort_reset_region(L.sort_ws, B, N, K, &zf.z1, &zf.n1);
   update_control_region(L.upd_ws, B, N, D, &zf.z3, &zf.n3);
+  // Shift slots: where the update fuses the finalize nothing else uses the
+  // sums region, so it holds as many as fit (one slot always does: slices
+  // of the workspace are whole 256-byte blocks); otherwise one slot per
+  // iteration (raised by launch_finalize).
+  const bool fuses = update_fuses_finalize(D);
+  int nslots = 1;
+  while (nslots < kShiftSlots && 2 * nslots * kShiftStride <= B * K * D)
+    nslots *= 2;
+  if (!fuses) nslots = 1;
   if (check) {
-    zf.z2 = L.shift;
-    zf.n2 = max_iters;
+    zf.z2 = fuses ? L.sums : L.shift;
+    zf.n2 = fuses ? (int64_t)nslots * kShiftStride : max_iters;
   }
   int rc = launch_lloyd_prologue(init, centroids, L.c_sq, B * K, D, dtype, zf, s);
   if (!rc && L.x_sq) rc = launch_row_sqnorm(x, L.x_sq, B * N, D, dtype, nullptr, s);
@@ -573,7 +582,8 @@ int lloyd_run(const void* x, const void* init, void* centroids,
     // The update finalizes the centroids itself when D <= 512 (no sums /
     // counts round trip); otherwise finalize runs as its own kernel.  Short
     // rows take the sort-free update: one launch, the same bits.
-    const UpdateFinalize fin{centroids, L.c_sq, check ? L.shift + it : nullptr};
+    float* const shift = !check ? nullptr : fuses ? L.sums : L.shift + it;
+    const UpdateFinalize fin{centroids, L.c_sq, shift, nslots};
     bool fused = false;
     if (!rc && scan) {
       rc = launch_update_scan(x, cluster_ids, B, N, K, D, dtype, L.upd_ws,
@@ -589,9 +599,9 @@ int lloyd_run(const void* x, const void* init, void* centroids,
                          &fused, it);
     if (!rc && !fused)
       rc = launch_finalize(L.sums, L.counts, centroids, centroids, L.c_sq,
-                           check ? L.shift + it : nullptr, B, K, D, dtype, ctrl,
-                           s);
-    if (!rc && check) rc = launch_converge_check(L.shift, it, tol, L.ctrl, s);
+                           shift, B, K, D, dtype, ctrl, s);
+    if (!rc && check)
+      rc = launch_converge_check(shift, nslots, it, tol, L.ctrl, s);
     if (rc) return rc;
   }
   if (!check && n_iters_dev) rc = launch_fill_i32(n_iters_dev, max_iters, 1, s);

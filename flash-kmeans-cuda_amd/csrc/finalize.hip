@@ -132,12 +132,24 @@ lloyd_prologue_kernel(const typename Elem<DT>::T* __restrict__ init,
 }
 
 // ctrl[0] = converged flag, ctrl[1] = iterations run.  Runs after the
-// finalize of iteration `it`, single thread.
-__global__ void converge_check_kernel(const float* shift, int it, float tol,
-                                      int32_t* ctrl) {
+// finalize of iteration `it`, one wave.  The slots are compared as the bits
+// they were raised with (a NaN shift is the largest and never below tol).
+__global__ void __launch_bounds__(64)
+converge_check_kernel(float* __restrict__ shift, int nslots, int it, float tol,
+                      int32_t* __restrict__ ctrl) {
   if (ctrl[0] != 0) return;
-  ctrl[1] = it + 1;
-  if (shift[it] < tol) ctrl[0] = 1;
+  uint32_t m = 0;
+  for (int i = threadIdx.x; i < nslots; i += 64) {
+    m = max(m, __float_as_uint(shift[i * kShiftStride]));
+    shift[i * kShiftStride] = 0.f;
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1)
+    m = max(m, (uint32_t)__shfl_xor((int)m, off, 64));
+  if (threadIdx.x == 0) {
+    ctrl[1] = it + 1;
+    if (__uint_as_float(m) < tol) ctrl[0] = 1;
+  }
 }
 
 unsigned grid_for(int64_t n) {
@@ -240,10 +252,10 @@ int launch_iota_i32(int32_t* p, int64_t B, int64_t N, hipStream_t s) {
   return check_launch("iota_i32");
 }
 
-int launch_converge_check(const float* shift, int it, float tol, int32_t* ctrl,
-                          hipStream_t s) {
-  hipLaunchKernelGGL(converge_check_kernel, dim3(1), dim3(1), 0, s, shift, it,
-                     tol, ctrl);
+int launch_converge_check(float* shift, int nslots, int it, float tol,
+                          int32_t* ctrl, hipStream_t s) {
+  hipLaunchKernelGGL(converge_check_kernel, dim3(1), dim3(64), 0, s, shift,
+                     nslots, it, tol, ctrl);
   return check_launch("converge_check");
 }
 

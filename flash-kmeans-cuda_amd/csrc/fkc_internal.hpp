@@ -104,11 +104,24 @@ size_t update_workspace_bytes(int64_t B, int64_t N, int64_t D);
 // centroids are written in place to `cent`, their squared norms to `c_sq`,
 // the max shift to `shift` (may be null), so no sums/counts round trip and
 // no finalize launch are needed.
+//
+// The shift is kept in nslots (a power of two) slots, kShiftStride floats
+// apart, bin k of batch row b raising slot (b * K + k) mod nslots; their
+// maximum is the shift.  With one slot every bin's atomic max meets the same
+// cache line: at (8, 65536, 1024, 64) bf16 with a tolerance update_runs took
+// 56.5 us and update_merge 46.7, about 36 and 40 us of it waiting for one
+// another; a call of 12 iterations 2302 -> 1335 us with 256 slots.
 struct UpdateFinalize {
   void* cent;
   float* c_sq;
   float* shift;
+  int nslots;
 };
+constexpr int kShiftStride = 16;  // floats: one 64-byte line per slot
+constexpr int kShiftSlots = 256;  // at most
+// Whether the update fuses the finalize for rows of D columns in overwrite
+// mode (else it leaves sums and counts for launch_finalize).
+bool update_fuses_finalize(int64_t D);
 // fin: optional fused finalize; *fused (may be null) reports whether it was
 // applied (it needs D <= 512); when not, the caller runs launch_finalize.
 // seq >= 0 (overwrite mode only): the number of earlier calls on this
@@ -169,8 +182,10 @@ int launch_lloyd_prologue(const void* init, void* cent, float* c_sq,
 int launch_iota_i32(int32_t* p, int64_t B, int64_t N, hipStream_t s);
 int launch_fill_f32(float* p, float v, int64_t n, hipStream_t s);
 int launch_fill_f64(double* p, double v, int64_t n, hipStream_t s);
-int launch_converge_check(const float* shift, int it, float tol, int32_t* ctrl,
-                          hipStream_t s);
+// Compares the maximum of the shift slots of iteration `it` to tol and
+// clears the slots for the next iteration.
+int launch_converge_check(float* shift, int nslots, int it, float tol,
+                          int32_t* ctrl, hipStream_t s);
 
 // FKC_ASSIGN_FORCE_SAFE=1|true: route every dtype to the fp32 VALU kernel.
 bool force_safe_assign();

@@ -154,7 +154,15 @@ template <typename T>
 struct FinArgs {
   T* cent;          // (B, K, D) centroids, updated in place; null: not fused
   float* c_sq;      // (B, K) next iteration's c_sq
-  float* shift;     // this iteration's max shift (float bits), may be null
+  float* shift;     // this iteration's shift slots (float bits), may be null
+  int smask;        // shift slots - 1
+
+  // The slot that row `bin` (b * K + k) raises.
+  __device__ float* slot(size_t bin) const {
+    return shift == nullptr
+               ? nullptr
+               : shift + ((uint32_t)bin & (uint32_t)smask) * kShiftStride;
+  }
 };
 
 // The lanes of one wave wrote `row` in LDS; make the writes visible to the
@@ -174,7 +182,8 @@ __device__ inline void finish_norms(float sq, float sh, float* csq,
   if (lane == 0) *csq = sq;
   if (shift != nullptr) {
     sh = row_sum(sh);
-    if (lane == 0)
+    // A row that did not move cannot raise the maximum.
+    if (lane == 0 && sh != 0.f)
       atomicMax(reinterpret_cast<unsigned int*>(shift), __float_as_uint(sqrtf(sh)));
   }
 }
@@ -461,7 +470,7 @@ update_runs_kernel(const typename Elem<DT>::T* __restrict__ x,
           RC::store(crow + col[i], nv);
         }
       finish_norms(sq, sh, fin.c_sq + (size_t)b * K + id,
-                   pref ? fin.shift : nullptr, lane);
+                   fin.slot((size_t)b * K + id), lane);
     } else if ((uint32_t)id < (uint32_t)K) {
       float* dst = sb + (size_t)id * D;
 #pragma unroll
@@ -841,7 +850,8 @@ update_merge_kernel(const float* __restrict__ part,
   if (fused) {
     wave_lds_sync();
     finalize_row<DT>(fin_row[wave], len, fin.cent + ((size_t)b * K + id) * D,
-                     fin.c_sq + (size_t)b * K + id, fin.shift, D, lane);
+                     fin.c_sq + (size_t)b * K + id,
+                     fin.slot((size_t)b * K + id), D, lane);
     return;
   }
   if (lane == 0) {
@@ -1103,7 +1113,8 @@ update_scan_kernel(const typename Elem<DT>::T* __restrict__ x,
     wave_lds_sync();
     const int id = k0 + j;
     finalize_row<DT>(s_row[wave], cnt, fin.cent + ((size_t)b * K + id) * D,
-                     fin.c_sq + (size_t)b * K + id, fin.shift, D, lane);
+                     fin.c_sq + (size_t)b * K + id,
+                     fin.slot((size_t)b * K + id), D, lane);
     wave_lds_sync();
   };
 
@@ -1256,7 +1267,8 @@ update_scan_kernel(const typename Elem<DT>::T* __restrict__ x,
       if (wave == 0)
         merge_finalize<DT>(s_part, (S1 - 1) / ur - S0 / ur, S1 - S0,
                            fin.cent + ((size_t)b * K + k0) * D,
-                           fin.c_sq + (size_t)b * K + k0, fin.shift, D, lane);
+                           fin.c_sq + (size_t)b * K + k0,
+                           fin.slot((size_t)b * K + k0), D, lane);
       return;
     }
   }
@@ -1434,7 +1446,7 @@ int launch_scan_t(const void* x, const int32_t* ids, const UpdateBufs& w,
                   int vec4, const UpdateFinalize& f, const int32_t* ctrl,
                   hipStream_t s) {
   using T = typename Elem<DT>::T;
-  FinArgs<T> fa{static_cast<T*>(f.cent), f.c_sq, f.shift};
+  FinArgs<T> fa{static_cast<T*>(f.cent), f.c_sq, f.shift, f.nslots - 1};
   dim3 grid((unsigned)((K + kpw - 1) / kpw), (unsigned)B);
   // Two register budgets for the row's labels: rows up to 8192 hold two
   // quads per thread, longer ones SCAN_UMAX; one owned label per workgroup
@@ -1489,6 +1501,12 @@ int64_t scan_kpw(int64_t B, int64_t K) {
 
 }  // namespace
 
+// Finalize fuses when a whole row fits one wave's column slices and LDS row
+// buffer (then grid.z == 1): even D <= 512, odd D <= 256.
+bool update_fuses_finalize(int64_t D) {
+  return D <= FIN_DMAX && D <= (int64_t)64 * runs_vec(D) * runs_ni(D);
+}
+
 size_t update_workspace_bytes(int64_t B, int64_t N, int64_t D) {
   return carve_update(nullptr, B, N, D).used;
 }
@@ -1527,30 +1545,31 @@ int launch_update(const void* x, const int32_t* perm,
   if (seq >= 0 && !overwrite)
     return fail(FKC_ERR_INVALID, "centroid_update: a sequenced call overwrites");
   const UpdateBufs w = carve_update(ws, B, N, D);
-  // Finalize fuses when a whole row fits one wave's column slices and LDS
-  // row buffer (D <= 512; then grid.z == 1) and every label is valid.
+  // (Overwrite mode: every label is valid.)
   const bool fuse = fin != nullptr && fin->cent != nullptr && overwrite &&
-                    D <= FIN_DMAX &&
-                    D <= (int64_t)64 * runs_vec(D) * runs_ni(D);
+                    update_fuses_finalize(D);
   if (fused) *fused = fuse;
   switch (dtype) {
     case FKC_F32: {
       FinArgs<float> f{fuse ? static_cast<float*>(fin->cent) : nullptr,
-                       fuse ? fin->c_sq : nullptr, fuse ? fin->shift : nullptr};
+                       fuse ? fin->c_sq : nullptr, fuse ? fin->shift : nullptr,
+                   fuse ? fin->nslots - 1 : 0};
       return launch_update_t<FKC_F32>(x, perm, ids_sorted, sums, counts, w, B,
                                       N, K, D, overwrite, seq, f, ctrl, s);
     }
     case FKC_F16: {
       using T = typename Elem<FKC_F16>::T;
       FinArgs<T> f{fuse ? static_cast<T*>(fin->cent) : nullptr,
-                   fuse ? fin->c_sq : nullptr, fuse ? fin->shift : nullptr};
+                   fuse ? fin->c_sq : nullptr, fuse ? fin->shift : nullptr,
+                   fuse ? fin->nslots - 1 : 0};
       return launch_update_t<FKC_F16>(x, perm, ids_sorted, sums, counts, w, B,
                                       N, K, D, overwrite, seq, f, ctrl, s);
     }
     case FKC_BF16: {
       using T = typename Elem<FKC_BF16>::T;
       FinArgs<T> f{fuse ? static_cast<T*>(fin->cent) : nullptr,
-                   fuse ? fin->c_sq : nullptr, fuse ? fin->shift : nullptr};
+                   fuse ? fin->c_sq : nullptr, fuse ? fin->shift : nullptr,
+                   fuse ? fin->nslots - 1 : 0};
       return launch_update_t<FKC_BF16>(x, perm, ids_sorted, sums, counts, w, B,
                                        N, K, D, overwrite, seq, f, ctrl, s);
     }
@@ -1563,8 +1582,7 @@ bool update_scan_ok(int64_t B, int64_t N, int64_t K, int64_t D) {
   const int o = update_scan_override();
   if (o == 0) return false;
   if (B < 1 || N < 1 || N > SCAN_NMAX || K < 1 || K > 65535) return false;
-  if (D < 1 || D > FIN_DMAX || D > (int64_t)64 * runs_vec(D) * runs_ni(D))
-    return false;
+  if (D < 1 || !update_fuses_finalize(D)) return false;
   if (scan_kpw(B, K) > SCAN_KPW) return false;
   // Taken on its own for every row it can hold, where it measured faster
   // than the three launches it replaces (loop time per iteration, same box,

@@ -209,6 +209,35 @@ def test_tol_stops_at_the_oracles_iteration():
     assert torch.equal(it, _T(init, "bf16")), "init_centroids was modified"
 
 
+@pytest.mark.parametrize("B,N,K,D", [
+    (1, 3000, 3, 1),       # one shift slot
+    (1, 3000, 2, 17),      # two slots, odd width
+    (2, 40000, 300, 64),   # every slot, raised by the run and the merge kernel
+    (1, 9000, 40, 128),    # sort-free update
+    (1, 40000, 30, 301),   # finalize not fused: one slot per iteration
+])
+def test_tol_stop_over_shift_slots(B, N, K, D):
+    """The tolerance meets the maximum over every shift slot: for a tol
+    between two successive record lows of the shift (recomputed from the
+    centroids of runs of 1, 2, ... iterations) the loop stops at the lower
+    one's iteration with the bits of a tol = 0 run of that length.  One NaN
+    centroid row keeps the shift NaN, and the loop runs to the end."""
+    from flash_kmeans_cuda import batch_kmeans_Euclid
+    g = torch.Generator(device="cuda").manual_seed(N + K + D)
+    x = torch.randn(B, N, D, device="cuda", generator=g)
+    init = x[:, :K].contiguous()
+    cs = [init] + [batch_kmeans_Euclid(x, K, max_iters=i, init_centroids=init)[1] for i in range(1, 13)]
+    sh = [(b.double() - a.double()).norm(dim=-1).max().item() for a, b in zip(cs, cs[1:])]
+    i = next(j for j in range(1, 12) if 0 < 1.02 * sh[j] <= min(sh[:j]))
+    tol = (sh[i] * min(sh[:i])) ** 0.5
+    ids, c, n = batch_kmeans_Euclid(x, K, max_iters=40, tol=tol, init_centroids=init)
+    assert n == i + 1, (n, i, sh)
+    ref = batch_kmeans_Euclid(x, K, max_iters=n, init_centroids=init)
+    assert torch.equal(ids, ref[0]) and torch.equal(c, ref[1])
+    x[0, 0] = float("nan")
+    assert batch_kmeans_Euclid(x, K, max_iters=4, tol=1e30, init_centroids=x[:, :K].contiguous())[2] == 4
+
+
 @pytest.mark.parametrize("cfg_name,N", [("c3", 65536), ("c2", 32768), ("c4", 8192),
                                         ("c5", 131072)])
 def test_loop_sort_paths_agree(monkeypatch, cfg_name, N):

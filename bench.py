@@ -50,7 +50,7 @@ sys.path.insert(0, os.path.join(HERE, "flash-kmeans-cuda_amd"))
 sys.path.insert(0, HERE)
 
 PEAK_TFLOPS_F16 = 2500.0          # MI355X dense fp16/bf16 MFMA
-PEAK_TFLOPS_F32 = 157.3           # MI355X fp32 (the fp32 route runs on the VALU)
+PEAK_TFLOPS_F32 = 157.3           # MI355X fp32 (matrix and packed vector rate)
 METRIC_C5 = "assign TFLOPS + end-to-end ms/iter at (1,524K,8192,128) fp16, 1 MI355X"
 PROFILE_PERIOD = 5                # event-time the assign of one timed iteration in 5
 PEAK_HBM_GBS = 8000.0
@@ -278,7 +278,7 @@ def _gemm_peak() -> int:
 
 def _ideal_ms(cfg) -> tuple[float, float, float]:
     """(assign flops, bytes moved per iteration, ideal ms per iteration) from
-    the algorithmic work: 2BNKD flops at the MFMA peak (VALU fp32 peak for
+    the algorithmic work: 2BNKD flops at the MFMA peak (fp32 peak for
     fp32) plus the iteration's bytes at the HBM peak.  Bytes: assign
     s*BND + s*BKD + 4BK + 4BN; sort, update, finalize, c_sq
     s*BND + 20BN + (3s+8)*BKD + 16BK."""

@@ -48,7 +48,7 @@ SOURCE_FLAGS = {"assign_mfma.hip": ["-fno-honor-nans"]}
 
 KERNEL_SOURCES = [
     "assign_mfma.hip",
-    "assign_valu.hip",
+    "assign_f32.hip",
     "label_sort.hip",
     "update.hip",
     "finalize.hip",

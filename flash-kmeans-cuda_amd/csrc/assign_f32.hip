@@ -1,0 +1,659 @@
+// fp32 assignment on the matrix cores, and row squared norms.
+//
+// The labels are those of the reference's tensor-core-free kernel
+// (flash_kmeans_cuda/csrc/assign/assign_safe.cu:38-81): for each point,
+//     dist_k = max(0, x_sq + c_sq[k] - 2 * <x, c_k>)      (assign_common.cuh:33-36)
+// with the dot product accumulated in fp32 as one fused multiply-add chain in
+// feature order, and the strict-< running minimum that keeps the lowest k on
+// ties (assign_common.cuh:23-28).  It serves fp32 inputs, fp16/bf16 with
+// D % 8 != 0 or D > 512, and FKC_ASSIGN_FORCE_SAFE (api.cpp:12-25).
+//
+// v_mfma_f32_16x16x4_f32 and v_mfma_f32_32x32x2_f32 add their products to
+// the accumulator as a chain of fused multiply-adds in k order (a probe
+// compared 2.5 million results, subnormals, infinities and NaN among them,
+// with fmaf on the host: no bit differed), so a sequence of them over the
+// features gives the chain's bits at the matrix cores' fp32 rate (133 and 149
+// TFLOP/s measured in registers alone; 78 is the vector peak without packed
+// instructions).
+//
+// Operands: A = M centroids x 64 / M features, B = as many features x M
+// points, so lane l holds centroid (A) or point (B) l % M.  Both are loaded
+// as quads of four consecutive features, lane group l / M the (l / M)-th
+// quad of a group of 4 * 64 / M features, and transposed over the lane groups
+// (v_permlane16_swap, v_permlane32_swap) into the operands of the group's
+// four steps.  The points' operands stay in registers for the whole scan
+// over K; the centroids' quads stream from the caches straight into
+// registers up to eight groups ahead, with neither LDS nor barriers.  One
+// quad feeds 4 * PT MFMAs, so a CU asks its L1 for at most 32 bytes a cycle.
+//
+// Bound by the matrix pipe and, on top of it, the vector instructions: fp32
+// MFMAs and vector work hardly overlap here (at (131072, 1024, 128), timing
+// copies without fold, loads and transposes ran 145 TFLOP/s, with them 110
+// to 115), so the fold is five instructions per score.  Measured against the
+// vector kernel this replaced, same labels: (1, 131072, 1024, 128) fp32 897
+// -> 300 us, (1, 8192, 256, 128) 45 -> 13, (1, 1000, 1000, 512) 614 -> 78,
+// (1, 100000, 300, 37) fp16 81 -> 39.  Staging the centroids through LDS in
+// operand order (no transposes) gained at most 5% at large N and lost at
+// small; folding a tile under the next one's MFMAs gained nothing.
+#include "device_util.hpp"
+#include "fkc_internal.hpp"
+
+#include <float.h>
+
+namespace fkc {
+
+int launch_assign_mfma(const void* x, const void* c, const float* c_sq,
+                       int32_t* ids, int64_t B, int64_t N, int64_t K,
+                       int64_t D, int dtype, const int32_t* ctrl,
+                       hipStream_t s, hipEvent_t ev0, hipEvent_t ev1,
+                       void* ws, size_t ws_bytes);
+
+namespace {
+
+constexpr int FT = 256;  // threads: four waves
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+
+// Four consecutive elements of a row.  Rows start wherever the caller's
+// tensor and D put them, so the loads ask for element alignment only.
+template <int DT>
+struct Quad {
+  typedef uint16_t Raw __attribute__((ext_vector_type(4), aligned(2)));
+  __device__ static f32x4 cvt(Raw r) {
+    typename Elem<DT>::T e[4];
+    const uint16_t h[4] = {r[0], r[1], r[2], r[3]};
+    __builtin_memcpy(e, h, 8);
+    return f32x4{Elem<DT>::load(e[0]), Elem<DT>::load(e[1]),
+                 Elem<DT>::load(e[2]), Elem<DT>::load(e[3])};
+  }
+};
+template <>
+struct Quad<FKC_F32> {
+  typedef float Raw __attribute__((ext_vector_type(4), aligned(4)));
+  __device__ static f32x4 cvt(Raw r) { return f32x4{r[0], r[1], r[2], r[3]}; }
+};
+
+// Features d .. d + 3 of a row of D.  whole: all four exist (d + 3 < D);
+// else those at D and after read as zero, which adds nothing to a chain.
+template <int DT>
+__device__ inline typename Quad<DT>::Raw load_quad(
+    const typename Elem<DT>::T* row, int d, int D, bool whole) {
+  using Raw = typename Quad<DT>::Raw;
+  if (whole) return *reinterpret_cast<const Raw*>(row + d);
+  Raw r;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    typename Elem<DT>::T v = row[min(d + e, D - 1)];
+    if constexpr (DT == FKC_F32) {
+      r[e] = d + e < D ? v : 0.f;
+    } else {
+      uint16_t h;
+      __builtin_memcpy(&h, &v, 2);
+      r[e] = d + e < D ? h : (uint16_t)0;
+    }
+  }
+  return r;
+}
+
+// The two instruction shapes: M x M scores, FG features per group of quads
+// (64 / M lane groups of four), four steps per group.
+template <int M>
+struct Shape;
+
+template <>
+struct Shape<16> {
+  static constexpr int FG = 16, R = 4;
+  typedef float Acc __attribute__((ext_vector_type(4)));
+  __device__ static Acc mfma(float a, float b, Acc c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+  }
+  // 4 x 4 transpose over the lane groups of 16: in, lane group q holds
+  // features 4 q + e of the group in register e; out, it holds feature
+  // 4 s + q in register s, the operand of step s.
+  __device__ static void steps(f32x4 v, float (&o)[4]) {
+    const u32x2 a = __builtin_amdgcn_permlane16_swap(
+        __float_as_uint(v[0]), __float_as_uint(v[1]), false, false);
+    const u32x2 b = __builtin_amdgcn_permlane16_swap(
+        __float_as_uint(v[2]), __float_as_uint(v[3]), false, false);
+    const u32x2 lo = __builtin_amdgcn_permlane32_swap(a[0], b[0], false, false);
+    const u32x2 hi = __builtin_amdgcn_permlane32_swap(a[1], b[1], false, false);
+    o[0] = __uint_as_float(lo[0]);
+    o[1] = __uint_as_float(hi[0]);
+    o[2] = __uint_as_float(lo[1]);
+    o[3] = __uint_as_float(hi[1]);
+  }
+  // Accumulator register r of lane group q holds centroid row(r) + 4 q.
+  __device__ static constexpr int row(int r) { return r; }
+};
+
+template <>
+struct Shape<32> {
+  static constexpr int FG = 8, R = 16;
+  typedef float Acc __attribute__((ext_vector_type(16)));
+  __device__ static Acc mfma(float a, float b, Acc c) {
+    return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
+  }
+  // In, half q of the wave holds features 4 q + e in register e; out, it
+  // holds feature 2 s + q in register s.
+  __device__ static void steps(f32x4 v, float (&o)[4]) {
+    const u32x2 a = __builtin_amdgcn_permlane32_swap(
+        __float_as_uint(v[0]), __float_as_uint(v[1]), false, false);
+    const u32x2 b = __builtin_amdgcn_permlane32_swap(
+        __float_as_uint(v[2]), __float_as_uint(v[3]), false, false);
+    o[0] = __uint_as_float(a[0]);
+    o[1] = __uint_as_float(b[0]);
+    o[2] = __uint_as_float(a[1]);
+    o[3] = __uint_as_float(b[1]);
+  }
+  __device__ static constexpr int row(int r) { return 8 * (r / 4) + r % 4; }
+};
+
+// Where a wave's work lies: ks (1, 2 or 4) waves of the workgroup share one
+// group of points and take every ks-th tile of 16 centroids.
+struct WaveWork {
+  int wave, kpart, n0;
+  __device__ WaveWork(int ks, int pts) {
+    wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    kpart = wave & (ks - 1);
+    const int per = 4 / ks;  // point groups of the workgroup
+    n0 = (blockIdx.x * per + wave / ks) * pts;
+  }
+};
+
+// c_sq of the centroids whose scores a lane holds of the block at k0 (row
+// K - 1 again past K).
+template <int M>
+__device__ inline void load_csq(const float* qb, int k0, int q, int K,
+                                float (&cq)[Shape<M>::R]) {
+#pragma unroll
+  for (int r = 0; r < Shape<M>::R; ++r)
+    cq[r] = qb[min(k0 + Shape<M>::row(r) + 4 * q, K - 1)];
+}
+
+// The scores a lane holds of one block (one point, centroid rows rising with
+// r) folded into its running minimum; strict < keeps the first.  best starts
+// at FLT_MAX and stays >= 0, so the median of dist, 0 and best is
+// min(max(dist, 0), best), and a NaN distance counts as 0 as the chain's
+// clamp has it.  bidx lacks the lane group's 4 q until the end: the index is
+// then wave-uniform and costs no vector instruction.
+template <int M, bool WHOLE>
+__device__ inline void fold_dist(const typename Shape<M>::Acc& acc, float xs,
+                                 const float (&cq)[Shape<M>::R], int k0, int q,
+                                 int K, float& best, int& bidx) {
+#pragma unroll
+  for (int r = 0; r < Shape<M>::R; ++r) {
+    const int k = k0 + Shape<M>::row(r);
+    const float dist = fmaf(-2.0f, acc[r], xs + cq[r]);
+    float nb = __builtin_amdgcn_fmed3f(dist, 0.f, best);
+    if constexpr (!WHOLE) nb = k + 4 * q < K ? nb : best;
+    bidx = nb < best ? k : bidx;
+    best = nb;
+  }
+}
+
+// fold_dist over a wave's PT point tiles.
+template <int M, int PT>
+__device__ inline void fold_tile(const typename Shape<M>::Acc (&acc)[PT],
+                                 const float (&xs)[PT],
+                                 const float (&cq)[Shape<M>::R], int k0, int q,
+                                 int K, float (&best)[PT], int (&bidx)[PT]) {
+  if (k0 + M <= K) {
+#pragma unroll
+    for (int p = 0; p < PT; ++p)
+      fold_dist<M, true>(acc[p], xs[p], cq, k0, q, K, best[p], bidx[p]);
+  } else {
+#pragma unroll
+    for (int p = 0; p < PT; ++p)
+      fold_dist<M, false>(acc[p], xs[p], cq, k0, q, K, best[p], bidx[p]);
+  }
+}
+
+// Merge the lane groups of each point, then the ks waves that share them
+// (smaller distance, then smaller index), and store the labels.
+template <int M, int PT>
+__device__ inline void merge_store(float (&best)[PT], int (&bidx)[PT], int ks,
+                                   const WaveWork& w, int32_t* ids, int N) {
+  static_assert(M * PT <= 64, "one point per lane");
+  __shared__ float s_best[4][M * PT];
+  __shared__ int s_idx[4][M * PT];
+  const int lane = threadIdx.x & 63, q = lane / M;
+#pragma unroll
+  for (int p = 0; p < PT; ++p) {
+    // No score below FLT_MAX: index 0, as the scan starts.
+    bidx[p] = best[p] < FLT_MAX ? bidx[p] + 4 * q : 0;
+#pragma unroll
+    for (int off = M; off < 64; off <<= 1) {
+      const float ob = __shfl_xor(best[p], off, 64);
+      const int oi = __shfl_xor(bidx[p], off, 64);
+      if (ob < best[p] || (ob == best[p] && oi < bidx[p])) {
+        best[p] = ob;
+        bidx[p] = oi;
+      }
+    }
+  }
+  // Lane group q keeps point tile q: lane l then holds point n0 + l.
+  float b = best[0];
+  int i = bidx[0];
+#pragma unroll
+  for (int p = 1; p < PT; ++p) {
+    b = q == p ? best[p] : b;
+    i = q == p ? bidx[p] : i;
+  }
+  if (ks > 1) {
+    if (lane < M * PT) {
+      s_best[w.wave][lane] = b;
+      s_idx[w.wave][lane] = i;
+    }
+    __syncthreads();
+    if (w.kpart != 0) return;
+    if (lane < M * PT) {
+      for (int j = 1; j < ks; ++j) {
+        const float ob = s_best[w.wave + j][lane];
+        const int oi = s_idx[w.wave + j][lane];
+        if (ob < b || (ob == b && oi < i)) {
+          b = ob;
+          i = oi;
+        }
+      }
+    }
+  }
+  if (lane < M * PT && w.n0 + lane < N) ids[w.n0 + lane] = i;
+}
+
+// ||x_n||^2 of the point tiles' points: given, or as the chain of v * v.
+template <int DT, int M, int PT>
+__device__ inline void point_norms(const typename Elem<DT>::T* xb,
+                                   const float* x_sq, int n0, int N, int D,
+                                   float (&xs)[PT]) {
+  const int col = threadIdx.x % M;
+#pragma unroll
+  for (int p = 0; p < PT; ++p) {
+    const int n = min(n0 + M * p + col, N - 1);
+    if (x_sq != nullptr) {
+      xs[p] = x_sq[n];
+    } else {
+      xs[p] = 0.f;
+      for (int d = 0; d < D; ++d) {
+        const float v = Elem<DT>::load(xb[(size_t)n * D + d]);
+        xs[p] = fmaf(v, v, xs[p]);
+      }
+    }
+  }
+}
+
+// D <= 512.  M: instruction shape; G: feature groups a row takes (D <= FG G),
+// the first NF of them certainly whole; PT: M-point tiles per wave.
+template <int DT, int M, int G, int NF, int PT>
+__global__ void __launch_bounds__(FT, 2)
+assign_f32_kernel(const typename Elem<DT>::T* __restrict__ x,
+                  const typename Elem<DT>::T* __restrict__ c,
+                  const float* __restrict__ x_sq,
+                  const float* __restrict__ c_sq, int32_t* __restrict__ ids,
+                  int N, int K, int D, int ks,
+                  const int32_t* __restrict__ ctrl) {
+  using T = typename Elem<DT>::T;
+  using Raw = typename Quad<DT>::Raw;
+  using S = Shape<M>;
+  // Quads in flight: eight against two gained 15% at (131072, 1024, 128).
+  constexpr int PD = G < 8 ? G : 8;
+  if (loop_done(ctrl)) return;
+  const int lane = threadIdx.x & 63, col = lane % M, q = lane / M;
+  const int b = blockIdx.y;
+  const WaveWork w(ks, M * PT);
+  const T* xb = x + (size_t)b * N * D;
+  const T* cb = c + (size_t)b * K * D;
+  const float* qb = c_sq + (size_t)b * K;
+
+  const int nt = (K + M - 1) / M;
+  // Quad g of this lane's row of tile t (row K - 1 past K: such rows are
+  // loaded but never win).
+  auto load_c = [&](int t, int g) -> Raw {
+    const T* row = cb + (size_t)min(M * t + col, K - 1) * D;
+    return load_quad<DT>(row, S::FG * g + 4 * q, D, g < NF);
+  };
+  Raw ring[PD];
+#pragma unroll
+  for (int i = 0; i < PD; ++i) ring[i] = load_c(w.kpart, i);
+
+  float bx[PT][G][4];
+#pragma unroll
+  for (int p = 0; p < PT; ++p) {
+    const T* row = xb + (size_t)min(w.n0 + M * p + col, N - 1) * D;
+    Raw raw[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+      raw[g] = load_quad<DT>(row, S::FG * g + 4 * q, D, g < NF);
+#pragma unroll
+    for (int g = 0; g < G; ++g) S::steps(Quad<DT>::cvt(raw[g]), bx[p][g]);
+  }
+  float xs[PT], best[PT];
+  int bidx[PT];
+  point_norms<DT, M, PT>(xb, x_sq ? x_sq + (size_t)b * N : nullptr, w.n0, N, D, xs);
+#pragma unroll
+  for (int p = 0; p < PT; ++p) {
+    best[p] = FLT_MAX;
+    bidx[p] = 0;
+  }
+
+  for (int t = w.kpart; t < nt; t += ks) {
+    float cq[S::R];
+    load_csq<M>(qb, M * t, q, K, cq);
+    typename S::Acc acc[PT];
+#pragma unroll
+    for (int p = 0; p < PT; ++p)
+#pragma unroll
+      for (int r = 0; r < S::R; ++r) acc[p][r] = 0.f;
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      const Raw cur = ring[0];
+#pragma unroll
+      for (int i = 0; i + 1 < PD; ++i) ring[i] = ring[i + 1];
+      ring[PD - 1] = g + PD < G ? load_c(t, g + PD) : load_c(t + ks, g + PD - G);
+      float a[4];
+      S::steps(Quad<DT>::cvt(cur), a);
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int p = 0; p < PT; ++p) acc[p] = S::mfma(a[s], bx[p][g][s], acc[p]);
+    }
+    fold_tile<M, PT>(acc, xs, cq, M * t, q, K, best, bidx);
+  }
+  merge_store<M, PT>(best, bidx, ks, w, ids + (size_t)b * N, N);
+}
+
+// Any D (used above 512, where a point tile's operands no longer fit the
+// registers): both operands stream, and 4 x 4 blocks of 16 x 16 scores per
+// wave give each quad four uses.  (1, 20000, 500, 768) fp32 974 us with the
+// vector kernel, 289 with this one; fp16 2362 and 284.
+template <int DT>
+__global__ void __launch_bounds__(FT, 2)
+assign_f32_wide_kernel(const typename Elem<DT>::T* __restrict__ x,
+                       const typename Elem<DT>::T* __restrict__ c,
+                       const float* __restrict__ x_sq,
+                       const float* __restrict__ c_sq,
+                       int32_t* __restrict__ ids, int N, int K, int D, int ks,
+                       const int32_t* __restrict__ ctrl) {
+  using T = typename Elem<DT>::T;
+  using Raw = typename Quad<DT>::Raw;
+  using S = Shape<16>;
+  constexpr int M = 16, PT = 4, CT = 4;
+  if (loop_done(ctrl)) return;
+  const int lane = threadIdx.x & 63, col = lane % M, q = lane / M;
+  const int b = blockIdx.y;
+  const WaveWork w(ks, M * PT);
+  const T* xb = x + (size_t)b * N * D;
+  const T* cb = c + (size_t)b * K * D;
+  const float* qb = c_sq + (size_t)b * K;
+  float xs[PT], best[PT];
+  int bidx[PT];
+  point_norms<DT, M, PT>(xb, x_sq ? x_sq + (size_t)b * N : nullptr, w.n0, N, D, xs);
+  const T* xrow[PT];
+#pragma unroll
+  for (int p = 0; p < PT; ++p) {
+    best[p] = FLT_MAX;
+    bidx[p] = 0;
+    xrow[p] = xb + (size_t)min(w.n0 + M * p + col, N - 1) * D;
+  }
+  const int nfull = D / S::FG;
+  const int nt = (K + M * CT - 1) / (M * CT);
+  for (int t = w.kpart; t < nt; t += ks) {
+    const int k0 = M * CT * t;
+    const T* crow[CT];
+#pragma unroll
+    for (int j = 0; j < CT; ++j)
+      crow[j] = cb + (size_t)min(k0 + M * j + col, K - 1) * D;
+    S::Acc acc[CT][PT];
+#pragma unroll
+    for (int j = 0; j < CT; ++j)
+#pragma unroll
+      for (int p = 0; p < PT; ++p) acc[j][p] = S::Acc{0.f, 0.f, 0.f, 0.f};
+    Raw rx[PT], rc[CT];
+    auto fetch = [&](int g, bool whole) {
+#pragma unroll
+      for (int p = 0; p < PT; ++p)
+        rx[p] = load_quad<DT>(xrow[p], S::FG * g + 4 * q, D, whole);
+#pragma unroll
+      for (int j = 0; j < CT; ++j)
+        rc[j] = load_quad<DT>(crow[j], S::FG * g + 4 * q, D, whole);
+    };
+    auto score = [&](const Raw (&ux)[PT], const Raw (&uc)[CT]) {
+      float a[CT][4], bx[PT][4];
+#pragma unroll
+      for (int p = 0; p < PT; ++p) S::steps(Quad<DT>::cvt(ux[p]), bx[p]);
+#pragma unroll
+      for (int j = 0; j < CT; ++j) S::steps(Quad<DT>::cvt(uc[j]), a[j]);
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int j = 0; j < CT; ++j)
+#pragma unroll
+          for (int p = 0; p < PT; ++p)
+            acc[j][p] = S::mfma(a[j][s], bx[p][s], acc[j][p]);
+    };
+    fetch(0, true);  // D > 512: group 0 is whole
+    for (int g = 0; g < nfull; ++g) {
+      Raw ux[PT], uc[CT];
+#pragma unroll
+      for (int p = 0; p < PT; ++p) ux[p] = rx[p];
+#pragma unroll
+      for (int j = 0; j < CT; ++j) uc[j] = rc[j];
+      fetch(min(g + 1, nfull - 1), true);
+      score(ux, uc);
+    }
+    if (D % S::FG != 0) {
+      fetch(nfull, false);
+      score(rx, rc);
+    }
+#pragma unroll
+    for (int j = 0; j < CT; ++j) {
+      float cq[S::R];
+      load_csq<M>(qb, k0 + M * j, q, K, cq);
+      fold_tile<M, PT>(acc[j], xs, cq, k0 + M * j, q, K, best, bidx);
+    }
+  }
+  merge_store<M, PT>(best, bidx, ks, w, ids + (size_t)b * N, N);
+}
+
+template <int DT>
+__global__ void __launch_bounds__(256)
+row_sqnorm_kernel(const typename Elem<DT>::T* __restrict__ src,
+                  float* __restrict__ out, int64_t rows, int D,
+                  const int32_t* __restrict__ ctrl) {
+  using E = Elem<DT>;
+  if (loop_done(ctrl)) return;
+  const int lane = threadIdx.x & 63;
+  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= rows) return;
+  const typename E::T* r = src + row * D;
+  // Column order and reduction shared with the finalize kernels.
+  const int vec = row_vec(D);
+  float acc = 0.f;
+  for (int c = vec * lane; c < D; c += vec * 64) {
+    for (int v = 0; v < vec; ++v) {
+      const float f = E::load(r[c + v]);
+      acc = fmaf(f, f, acc);
+    }
+  }
+  acc = row_sum(acc);
+  if (lane == 0) out[row] = acc;
+}
+
+// The launch of a shape: instruction shape m, m-point tiles per wave (pt),
+// waves of a workgroup that share their points and split K (ks).
+struct F32Plan {
+  int m, pt, ks;
+};
+
+// 32 x 32 blocks step eight features at a time, 16 x 16 blocks sixteen: where
+// D's last sixteen are at most half used, 32 x 32 saves the padding
+// ((131072, 1000, D) fp32, 16 x 16 against 32 x 32: D = 24 103 / 79 us, 40
+// 132 / 110, 72 203 / 177, 104 261 / 246, 200 536 / 497); elsewhere 16 x 16
+// is as fast or faster (64 159 / 160, 96 223 / 228, 128 292 / 302, 160 413 /
+// 426) and wastes less of a small K.
+bool f32_has_m32(int64_t D) { return D <= 248 && (D + 7) / 8 % 2 == 1; }
+
+// The candidate with the least modelled time: waves per SIMD, rounded up,
+// times a wave's work in 16 x 16 blocks.  A wave's own start costs about two
+// 16-centroid tiles; fewer points per wave mean more centroid loads per MFMA
+// (factors measured at (131072, 1024, 128): four tiles 1, two 1.05, one 1.5);
+// one wave alone on a SIMD reaches 0.77 of what two do.
+F32Plan plan_f32(int64_t B, int64_t N, int64_t K, int64_t D) {
+  const int64_t simds = 4 * (int64_t)device_shape().cus;
+  F32Plan best{16, 1, 1};
+  double least = 0;
+  for (int m = 16; m <= 32; m *= 2) {
+    if (m == 32 && !f32_has_m32(D)) break;
+    const int u = m / 16;
+    const int64_t nt = (K + m - 1) / m;
+    const double groups = m == 16 ? 2 * ((D + 15) / 16) : (D + 7) / 8;
+    const int pt_max = (D <= 128 ? 4 : D <= 256 ? 2 : 1) / u;
+    for (int pt = pt_max; pt >= 1; pt >>= 1) {
+      const double reuse = pt * u >= 4 ? 1.0 : pt * u == 2 ? 1.05 : 1.5;
+      for (int ks = 1; ks <= 4 && ks <= nt; ks *= 2) {
+        const int64_t waves = B * ((N + m * pt - 1) / (m * pt)) * ks;
+        const double t = (double)((waves + simds - 1) / simds) *
+                         (waves <= simds ? 1.3 : 1.0) * pt * u * reuse *
+                         groups * ((double)((nt + ks - 1) / ks) * u + 2);
+        if (least == 0 || t < least) {
+          least = t;
+          best = {m, pt, ks};
+        }
+      }
+    }
+  }
+  return best;
+}
+
+template <int DT>
+int launch_f32_t(const void* x, const void* c, const float* x_sq,
+                 const float* c_sq, int32_t* ids, int64_t B, int64_t N,
+                 int64_t K, int64_t D, const int32_t* ctrl, hipStream_t s) {
+  using T = typename Elem<DT>::T;
+  F32Plan p{16, 4, 1};
+  if (D <= 512) {
+    p = plan_f32(B, N, K, D);
+  } else {
+    const int64_t want = 8 * (int64_t)device_shape().cus, nt = (K + 63) / 64;
+    while (p.ks < 4 && 2 * p.ks <= nt && B * ((N + 63) / 64) * p.ks < want)
+      p.ks *= 2;
+  }
+  const int64_t per = p.m * p.pt * (4 / p.ks);  // points per workgroup
+  const dim3 grid((unsigned)((N + per - 1) / per), (unsigned)B);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(FT), 0, s, static_cast<const T*>(x),
+                       static_cast<const T*>(c), x_sq, c_sq, ids, (int)N,
+                       (int)K, (int)D, p.ks, ctrl);
+    return check_launch("assign_f32");
+  };
+  if (D > 512) return go(assign_f32_wide_kernel<DT>);
+  // G feature groups cover D; the NF groups of the next smaller variant are
+  // certainly whole (all G where fp32 fills them exactly).  The points'
+  // operands take 128 registers at most, which leaves two waves per SIMD.
+#define FKC_F32_G(M, G, NF, PTMAX)                                           \
+  if (p.m == M && D <= Shape<M>::FG * G) {                                   \
+    if constexpr (DT == FKC_F32 && M == 16) {                                \
+      if (D == Shape<M>::FG * G) {                                           \
+        if (p.pt == 1) return go(assign_f32_kernel<DT, M, G, G, 1>);         \
+        if constexpr (PTMAX >= 2)                                            \
+          if (p.pt == 2) return go(assign_f32_kernel<DT, M, G, G, 2>);       \
+        if constexpr (PTMAX >= 4)                                            \
+          if (p.pt == 4) return go(assign_f32_kernel<DT, M, G, G, 4>);       \
+      }                                                                      \
+    }                                                                        \
+    if (p.pt == 1) return go(assign_f32_kernel<DT, M, G, NF, 1>);            \
+    if constexpr (PTMAX >= 2)                                                \
+      if (p.pt == 2) return go(assign_f32_kernel<DT, M, G, NF, 2>);          \
+    if constexpr (PTMAX >= 4)                                                \
+      if (p.pt == 4) return go(assign_f32_kernel<DT, M, G, NF, 4>);          \
+  }
+  FKC_F32_G(16, 1, 0, 4)
+  FKC_F32_G(16, 2, 1, 4)
+  FKC_F32_G(16, 3, 2, 4)
+  FKC_F32_G(16, 4, 3, 4)
+  FKC_F32_G(16, 5, 4, 4)
+  FKC_F32_G(16, 6, 5, 4)
+  FKC_F32_G(16, 7, 6, 4)
+  FKC_F32_G(16, 8, 7, 4)
+  FKC_F32_G(16, 10, 8, 2)
+  FKC_F32_G(16, 12, 10, 2)
+  FKC_F32_G(16, 14, 12, 2)
+  FKC_F32_G(16, 16, 14, 2)
+  FKC_F32_G(16, 20, 16, 1)
+  FKC_F32_G(16, 24, 20, 1)
+  FKC_F32_G(16, 28, 24, 1)
+  FKC_F32_G(16, 32, 28, 1)
+  FKC_F32_G(32, 1, 0, 2)
+  FKC_F32_G(32, 3, 2, 2)
+  FKC_F32_G(32, 5, 4, 2)
+  FKC_F32_G(32, 7, 6, 2)
+  FKC_F32_G(32, 9, 8, 2)
+  FKC_F32_G(32, 11, 10, 2)
+  FKC_F32_G(32, 13, 12, 2)
+  FKC_F32_G(32, 15, 14, 2)
+  FKC_F32_G(32, 17, 16, 1)
+  FKC_F32_G(32, 19, 18, 1)
+  FKC_F32_G(32, 21, 20, 1)
+  FKC_F32_G(32, 23, 22, 1)
+  FKC_F32_G(32, 25, 24, 1)
+  FKC_F32_G(32, 27, 26, 1)
+  FKC_F32_G(32, 29, 28, 1)
+  FKC_F32_G(32, 31, 30, 1)
+#undef FKC_F32_G
+  return fail(FKC_ERR_UNSUPPORTED, "assign_f32: no kernel for D = %lld",
+              (long long)D);
+}
+
+template <int DT>
+int launch_rowsq_t(const void* src, float* out, int64_t rows, int64_t D,
+                   const int32_t* ctrl, hipStream_t s) {
+  using T = typename Elem<DT>::T;
+  dim3 grid((unsigned)((rows + 3) / 4));
+  hipLaunchKernelGGL((row_sqnorm_kernel<DT>), grid, dim3(256), 0, s,
+                     static_cast<const T*>(src), out, rows, (int)D, ctrl);
+  return check_launch("row_sqnorm");
+}
+
+}  // namespace
+
+int launch_assign(const void* x, const void* c, const float* x_sq,
+                  const float* c_sq, int32_t* ids, int64_t B, int64_t N,
+                  int64_t K, int64_t D, int dtype, const int32_t* ctrl,
+                  hipStream_t s, hipEvent_t ev0, hipEvent_t ev1, void* ws,
+                  size_t ws_bytes) {
+  if (B == 0 || N == 0) return FKC_OK;
+  if (assign_uses_mfma(dtype, D))
+    return launch_assign_mfma(x, c, c_sq, ids, B, N, K, D, dtype, ctrl, s,
+                              ev0, ev1, ws, ws_bytes);
+  // The fp32 route marks its span with event records on the stream.
+  if (ev0 != nullptr) (void)hipEventRecord(ev0, s);
+  int rc = FKC_OK;
+  switch (dtype) {
+    case FKC_F32:
+      rc = launch_f32_t<FKC_F32>(x, c, x_sq, c_sq, ids, B, N, K, D, ctrl, s);
+      break;
+    case FKC_F16:
+      rc = launch_f32_t<FKC_F16>(x, c, x_sq, c_sq, ids, B, N, K, D, ctrl, s);
+      break;
+    case FKC_BF16:
+      rc = launch_f32_t<FKC_BF16>(x, c, x_sq, c_sq, ids, B, N, K, D, ctrl, s);
+      break;
+    default:
+      return fail(FKC_ERR_INVALID, "assign: unknown dtype %d", dtype);
+  }
+  if (ev1 != nullptr) (void)hipEventRecord(ev1, s);
+  return rc;
+}
+
+int launch_row_sqnorm(const void* src, float* out, int64_t rows, int64_t D,
+                      int dtype, const int32_t* ctrl, hipStream_t s) {
+  if (rows == 0) return FKC_OK;
+  switch (dtype) {
+    case FKC_F32: return launch_rowsq_t<FKC_F32>(src, out, rows, D, ctrl, s);
+    case FKC_F16: return launch_rowsq_t<FKC_F16>(src, out, rows, D, ctrl, s);
+    case FKC_BF16: return launch_rowsq_t<FKC_BF16>(src, out, rows, D, ctrl, s);
+  }
+  return fail(FKC_ERR_INVALID, "row_sqnorm: unknown dtype %d", dtype);
+}
+
+}  // namespace fkc

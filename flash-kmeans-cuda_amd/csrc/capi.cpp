@@ -210,7 +210,7 @@ static int dtype_ok(int dtype, const char* what) {
 namespace fkc {
 namespace {
 struct LoopBuffers {
-  float* x_sq = nullptr;   // only when the VALU assign route is taken
+  float* x_sq = nullptr;   // only when the fp32 assign route is taken
   float* c_sq = nullptr;
   int32_t* sorted = nullptr;
   int32_t* perm = nullptr;

@@ -187,7 +187,7 @@ int launch_fill_f64(double* p, double v, int64_t n, hipStream_t s);
 int launch_converge_check(float* shift, int nslots, int it, float tol,
                           int32_t* ctrl, hipStream_t s);
 
-// FKC_ASSIGN_FORCE_SAFE=1|true: route every dtype to the fp32 VALU kernel.
+// FKC_ASSIGN_FORCE_SAFE=1|true: route every dtype to the fp32 kernel.
 bool force_safe_assign();
 // ---------------------------------------------------------------- quality
 size_t quality_workspace_bytes(int64_t B, int64_t N, int64_t K);

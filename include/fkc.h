@@ -67,7 +67,7 @@ FKC_CAPI const char* fkc_version(void);
  *   - fp16/bf16 with D % 8 == 0 and D <= 512: MFMA kernel ranking
  *     c_sq[k] - 2<x,c_k> in fp32 (x_sq is not read; like the reference's
  *     raw-distance route, assign_sm80.cu:437-441, 687).
- *   - every other case, and FKC_ASSIGN_FORCE_SAFE=1: fp32 VALU kernel ranking
+ *   - every other case, and FKC_ASSIGN_FORCE_SAFE=1: fp32 kernel ranking
  *     max(0, x_sq + c_sq - 2<x,c>) (assign_safe.cu:55-80,
  *     assign_common.cuh:33-36).  x_sq may be NULL: then it is computed.
  * c_sq must hold the fp32 squared norms of the centroids as stored.

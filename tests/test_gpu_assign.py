@@ -330,6 +330,75 @@ def test_valu_resident_table_matches_tiled(monkeypatch, B, N, K, D, dtype):
     _check(x, c, dtype, got_r, max_frac=1e-3 if B * N >= 4096 else None)
 
 
+def _chain_labels(x, c, x_sq, c_sq):
+    """Labels of the fp32 route restated on the CPU: dot products as one
+    fused multiply-add chain in feature order (each step exact in 80-bit
+    arithmetic, then rounded to fp32), the clamped distance, the first
+    minimum below FLT_MAX.  x (n, D), c (K, D), all fp32 values."""
+    ld = np.longdouble
+    with np.errstate(invalid="ignore", over="ignore"):
+        acc = np.zeros((x.shape[0], c.shape[0]), np.float32)
+        for d in range(x.shape[1]):
+            acc = (ld(acc) + ld(x[:, d, None]) * ld(c[None, :, d])).astype(np.float32)
+        t = x_sq[:, None] + c_sq[None, :]
+        dist = (ld(t) - 2 * ld(acc)).astype(np.float32)
+        dist = np.where(dist > 0, dist, np.float32(0))
+    first = dist.argmin(1)
+    return np.where(dist.min(1) < np.finfo(np.float32).max, first, 0)
+
+
+FP32_CHAIN_CASES = [
+    # (B, N, K, D, dtype): single values, tiles of 16 and 32 points and
+    # centroids less, exactly and more than filled, feature groups of 8 and
+    # 16 whole and partial, rows of every load alignment, the widest resident
+    # row and the streamed ones, one and several waves per point group.
+    (1, 1, 1, 1, "f32"), (2, 17, 15, 3, "f32"), (1, 65, 16, 16, "f32"),
+    (3, 33, 17, 20, "f32"), (1, 1000, 64, 64, "f32"), (1, 4096, 64, 128, "f32"),
+    (1, 500, 100, 127, "f32"), (1, 300, 33, 129, "f32"), (1, 200, 70, 249, "f32"),
+    (1, 100, 65, 511, "f32"), (1, 100, 65, 512, "f32"), (1, 70, 129, 513, "f32"),
+    (2, 65, 64, 528, "f32"), (1, 140001, 70, 24, "f32"), (1, 262145, 33, 128, "f32"),
+    (1, 140001, 130, 37, "f16"), (2, 999, 40, 5, "bf16"), (1, 333, 50, 251, "bf16"),
+    (1, 129, 31, 640, "f16"),
+]
+
+
+@pytest.mark.parametrize("B,N,K,D,dtype", FP32_CHAIN_CASES)
+def test_fp32_route_is_the_fma_chain(B, N, K, D, dtype):
+    """Bit for bit, ties, NaN and infinities among them, with x_sq passed and
+    computed by the kernel (all points, or 300 of a large N)."""
+    from flash_kmeans_cuda import _C, synth
+    from flash_kmeans_cuda.ops import row_sqnorm
+    rng = np.random.default_rng(N + K + D)
+    xf = rng.standard_normal((B, N, D)).astype(np.float32)
+    cf = rng.standard_normal((B, K, D)).astype(np.float32)
+    xf[:, ::3] = np.round(xf[:, ::3])       # exact ties between rounded rows
+    cf[:, ::2] = np.round(cf[:, ::2])
+    if K > 2:
+        cf[:, K - 1] = cf[:, 1]
+    if N >= 100:
+        xf[:, 7, D // 2] = np.nan
+        xf[:, 11, 0] = np.inf
+        xf[:, 13] *= 1e4
+        cf[:, K // 2, D - 1] = -np.inf
+        xf[:, 17] = cf[:, 0]
+    xt, ct = synth.to_torch(O.from_f32(xf, dtype), dtype), synth.to_torch(O.from_f32(cf, dtype), dtype)
+    xs, cs = row_sqnorm(xt), row_sqnorm(ct)
+    got = _C.euclid_assign(xt, ct, xs, cs).cpu().numpy()
+    own = _C.euclid_assign(xt, ct, torch.empty(0, device="cuda"), cs).cpu().numpy()
+    pick = np.arange(N) if N <= 5000 else np.r_[0:100, N - 100:N, rng.integers(0, N, 100)]
+    for b in range(B):
+        xv, cv = xt[b].float().cpu().numpy()[pick], ct[b].float().cpu().numpy()
+        csb = cs[b].cpu().numpy()
+        ref = _chain_labels(xv, cv, xs[b].cpu().numpy()[pick], csb)
+        assert np.array_equal(got[b, pick], ref)
+        with np.errstate(invalid="ignore", over="ignore"):
+            sq = np.zeros(len(pick), np.float32)
+            for d in range(D):
+                v = np.longdouble(xv[:, d])
+                sq = (np.longdouble(sq) + v * v).astype(np.float32)
+        assert np.array_equal(own[b, pick], _chain_labels(xv, cv, sq, csb))
+
+
 def test_force_safe_env_routes_to_fp32_kernel(monkeypatch):
     x, c = _data(1, 2048, 128, 128, "f16", seed=21)
     monkeypatch.setenv("FKC_ASSIGN_FORCE_SAFE", "1")

@@ -127,7 +127,6 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 #define FKC_WHOLE_STAGE 1
 #endif
 
-constexpr int KC = 64;  // centroid rows per register-staged LDS stage
 constexpr int THREADS = 256;  // 4 waves
 
 template <int DT>
@@ -224,6 +223,12 @@ __device__ inline void progress_prio(int done, int total) {
     __builtin_amdgcn_s_setprio(0);
 }
 
+// Wide rows with twice the tiles: four up to D = 256, two up to 512 (at most
+// 128 point registers, two waves per SIMD).
+constexpr bool wide_pt(int ds2, int pt) {
+  return (pt == 4 && ds2 >= 5 && ds2 <= 8) || (pt == 2 && ds2 >= 9);
+}
+
 // DS2: 32-feature steps (padded width DP = 32*DS2 >= D); PT: 16-point tiles
 // per wave; PAD: D < DP, so segments past D read as zeros (a compile-time
 // flag: the unpadded variants carry no per-load condition); EXACT: track
@@ -237,7 +242,7 @@ __device__ inline void progress_prio(int done, int total) {
 template <int DT, int DS2, int PT, bool PAD, bool EXACT, bool SAVE,
           bool WHOLE = false>
 __global__ void __launch_bounds__(THREADS,
-                                  PT == 8 ? 2
+                                  (PT == 8 || wide_pt(DS2, PT)) ? 2
                                   : (SAVE && DS2 == 2) ? 3
                                   : (DS2 == 2 && PT <= 4) ? 4
                                   : (PT * DS2 <= 16 && DS2 <= 9) ? FKC_AB
@@ -259,6 +264,10 @@ assign_mfma_kernel(const uint16_t* __restrict__ x,
   const int k0 = blockIdx.z * kspan;
   K = min(Kall - k0, kspan);
   constexpr int DP = DS2 * 32;
+  constexpr bool WIDE = wide_pt(DS2, PT);
+  // Centroid rows per register-staged LDS stage (32 where 64 would leave a
+  // CU room for one workgroup only, and staging registers short).
+  constexpr int KC = WIDE && DS2 > 8 ? 32 : 64;
   constexpr int ROW = DP + 8;       // LDS row stride in 16-bit elements
   constexpr int SEGS = DP / 8;      // 16-byte segments per padded row
   constexpr int PIECES = KC * SEGS;
@@ -270,7 +279,8 @@ assign_mfma_kernel(const uint16_t* __restrict__ x,
   // Direct-to-LDS stages for unpadded power-of-two step counts (D = 32, 64,
   // 128, 256); measured faster than register staging at D = 64 and 128.
   constexpr bool DMA =
-      FKC_USE_DMA && !PAD && (DS2 == 1 || DS2 == 2 || DS2 == 4 || DS2 == 8);
+      FKC_USE_DMA && !PAD &&
+      (DS2 == 1 || DS2 == 2 || DS2 == 4 || DS2 == 8 || (DS2 == 16 && PT == 2));
 
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
@@ -351,7 +361,8 @@ assign_mfma_kernel(const uint16_t* __restrict__ x,
                          : DS2 == 1 ? 4 * FKC_KC_DMA
                          : DS2 == 2 ? 2 * FKC_KC_DMA
                          : DS2 <= 4 ? FKC_KC_DMA
-                                    : 64;
+                         : DS2 <= 8 ? 64
+                                    : 32;
     constexpr int KCD = (KCD0 * DP * 2) % (THREADS * 16) == 0 ? KCD0 : 64;
     constexpr int ROWB = DP * 2;
     constexpr int STAGE = KCD * ROWB;
@@ -461,7 +472,25 @@ assign_mfma_kernel(const uint16_t* __restrict__ x,
           }
           fold(acc, kb + 16 * t);
         }
-      } else if constexpr (PT == 8) {
+      } else if constexpr (DS2 > 8) {
+        // The fragments of a whole block (64 registers) do not fit beside
+        // the points: read step by step, as far ahead as registers allow.
+#pragma unroll
+        for (int t = 0; t < NTD; ++t) {
+          const f32x4 ci = *reinterpret_cast<const f32x4*>(lq + 16 * t + 4 * g);
+          const uint8_t* arow = lc + (16 * t + col) * ROWB;
+          f32x4 acc[PT];
+#pragma unroll
+          for (int s = 0; s < DS2; ++s) {
+            const u32x4 a =
+                *reinterpret_cast<const u32x4*>(arow + (((4 * s + g) ^ sw) * 16));
+#pragma unroll
+            for (int p = 0; p < PT; ++p)
+              acc[p] = mfma16<DT>(a, xr[p][s], s == 0 ? ci : acc[p]);
+          }
+          fold(acc, kb + 16 * t);
+        }
+      } else if constexpr (PT == 8 || WIDE) {
         // Eight tiles: the point registers leave no room for a second set
         // of accumulators, so each block is folded after its own MFMAs; the
         // next block's fragments are still read a block ahead, and the
@@ -724,26 +753,13 @@ assign_mfma_kernel(const uint16_t* __restrict__ x,
         base = obase;
       }
     }
-    // Every load of the re-score is issued before any of them is used:
+    // The loads of the re-score are issued before any of them is used:
     // unconditional, from rows clamped to K - 1 (a clamped row only stands
     // for a candidate past K, whose seed is -inf below), so the tile costs
     // one memory round trip rather than one per load.  Each lane loads its
-    // own point's four candidate rows (its segments of them) and their c_sq.
-    float cq[4];
-    u32x4 ar[4][DS2];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int kr = min(base + r, K - 1);
-      cq[r] = qb[kr];
-      const u32x4* crow = reinterpret_cast<const u32x4*>(cb + (size_t)kr * D);
-#pragma unroll
-      for (int s = 0; s < DS2; ++s) {
-        const int seg = 4 * s + g;
-        // Padded widths load an in-bounds segment and zero it past D.
-        const u32x4 v = crow[padded ? min(seg, dsegs - 1) : seg];
-        ar[r][s] = (!padded || seg < dsegs) ? v : u32x4{0u, 0u, 0u, 0u};
-      }
-    }
+    // own point's four candidate rows (its segments of them) and their c_sq;
+    // RB rows at a time where the points leave no registers for four.
+    constexpr int RB = !WIDE || DS2 == 5 ? 4 : DS2 <= 9 ? 2 : 1;
     // Only the diagonal of each chain is read: accumulator row i = col
     // (element e = col & 3 of the lane with g == col / 4) is point col
     // against its own candidate, and that lane loaded this very point's
@@ -753,16 +769,34 @@ assign_mfma_kernel(const uint16_t* __restrict__ x,
     const int e = col & 3;  // this lane's diagonal element when g == col/4
     float dv[4];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const float seed = base + r < K ? -0.5f * cq[r] : -INFINITY;
-      f32x4 acc = {seed, seed, seed, seed};
+    for (int r0 = 0; r0 < 4; r0 += RB) {
+      float cq[RB];
+      u32x4 ar[RB][DS2];
 #pragma unroll
-      for (int s = 0; s < DS2; ++s) acc = mfma16<DT>(ar[r][s], xr[p][s], acc);
-      float d = acc[0];
-      d = e == 1 ? acc[1] : d;
-      d = e == 2 ? acc[2] : d;
-      d = e == 3 ? acc[3] : d;
-      dv[r] = d;
+      for (int r = 0; r < RB; ++r) {
+        const int kr = min(base + r0 + r, K - 1);
+        cq[r] = qb[kr];
+        const u32x4* crow = reinterpret_cast<const u32x4*>(cb + (size_t)kr * D);
+#pragma unroll
+        for (int s = 0; s < DS2; ++s) {
+          const int seg = 4 * s + g;
+          // Padded widths load an in-bounds segment and zero it past D.
+          const u32x4 v = crow[padded ? min(seg, dsegs - 1) : seg];
+          ar[r][s] = (!padded || seg < dsegs) ? v : u32x4{0u, 0u, 0u, 0u};
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < RB; ++r) {
+        const float seed = base + r0 + r < K ? -0.5f * cq[r] : -INFINITY;
+        f32x4 acc = {seed, seed, seed, seed};
+#pragma unroll
+        for (int s = 0; s < DS2; ++s) acc = mfma16<DT>(ar[r][s], xr[p][s], acc);
+        float d = acc[0];
+        d = e == 1 ? acc[1] : d;
+        d = e == 2 ? acc[2] : d;
+        d = e == 3 ? acc[3] : d;
+        dv[r0 + r] = d;
+      }
     }
     int rr = 0;
     float m = dv[0];
@@ -1182,7 +1216,7 @@ constexpr MfmaLauncher entry(bool pad, bool exact, bool save, bool whole) {
         return &launch_mfma_t<DT, DS2, PT, false, false, false>;
     }
     return nullptr;
-  } else if constexpr (PT * DS2 * 4 <= 64) {
+  } else if constexpr (PT * DS2 * 4 <= 64 || wide_pt(DS2, PT)) {
     if (save) {
       // Saved-score fold: four tiles at D = 64 or 97..128, unpadded only.
       if constexpr (PT == 4 && (DS2 == 4 || DS2 == 2)) {
@@ -1192,8 +1226,10 @@ constexpr MfmaLauncher entry(bool pad, bool exact, bool save, bool whole) {
     }
     if constexpr (DS2 == 1 || DS2 == 2 || DS2 == 4 || DS2 == 8) {
       // One whole-table stage: exact index, unpadded, direct stages.
-      if (whole && exact && !pad)
-        return &launch_mfma_t<DT, DS2, PT, false, true, false, true>;
+      if constexpr (!wide_pt(DS2, PT)) {
+        if (whole && exact && !pad)
+          return &launch_mfma_t<DT, DS2, PT, false, true, false, true>;
+      }
     }
     if (exact)
       return pad ? &launch_mfma_t<DT, DS2, PT, true, true, false>
@@ -1207,7 +1243,8 @@ constexpr MfmaLauncher entry(bool pad, bool exact, bool save, bool whole) {
 
 // pt: 16-point tiles per wave (1, 2, 4, or 8 for unpadded D = 128 with the
 // re-score epilogue).  The 1/2/4 variants keep the point registers
-// (PT * DS2 * 4 VGPRs) at <= 64; the eight-tile one holds 128.
+// (PT * DS2 * 4 VGPRs) at <= 64; the eight-tile one and wide_pt's hold up to
+// 128.
 template <int DT, int DS2>
 MfmaLauncher by_pt(int pt, bool pad, bool exact, bool save, bool whole) {
   switch (pt) {
@@ -1256,9 +1293,21 @@ bool assign_uses_mfma(int dtype, int64_t D) {
 // (measured on MI355X's 256 CUs at N = 131072, K = 2048 and N = 65536,
 // K = 8192: four tiles on 512 / 256 workgroups beat two tiles on 1024 / 512
 // by 3% / 5%); eight tiles run 2 workgroups per CU and need two rounds of
-// them.
+// them.  Wide rows (D > 128) are bound by their LDS fragment reads: at
+// D = 256 two tiles read 128 bytes a cycle from LDS to keep the matrix cores
+// busy, all a CU has, four tiles half of it, so more tiles pay on fewer
+// workgroups.  Same-box fp16 assign times (us), tiles per wave 1 / 2 / 4:
+//   (49152, 2000, 160) 54 / 51 / 56      (49152, 2000, 256) 81 / 67 / 79
+//   (32768, 2000, 256) 50 / 49 / 78      (32768, 300, 256) 11 / 13 / 19
+//   (100000, 4096, 256) 302 / 245 / 224  (65536, 2048, 256) 96 / 74 / 80
+//   (262144, 2048, 256) 361 / 275 / 239  (262144, 2048, 160) 271 / 187 / 166
+// and 1 / 2 above D = 256, where one tile also runs one workgroup per CU:
+//   (16384, 2000, 512) 77 / 109          (24000, 2000, 512) 150 / 111
+//   (131072, 2048, 512) 602 / 289        (262144, 2048, 320) 783 / 379.
 static int64_t fill_wgs(int pt, int ds2, bool exact) {
   const int64_t cus = device_shape().cus;
+  if (ds2 >= 9 && pt == 2) return cus / 2 + 1;
+  if (ds2 >= 5 && pt >= 2) return cus + cus / 2;
   return (!exact && pt == 4 && ds2 == 4) ? cus : 4 * cus;
 }
 
@@ -1286,9 +1335,11 @@ static int choose_pt(int ds2, bool pad, bool exact, int64_t B, int64_t N,
                      int64_t K) {
   const int o = ntiles_override();
   if (o == 8 && pt8_ok(ds2, pad, exact)) return o;
-  if (o != 0 && o != 8 && o * ds2 * 4 <= 64) return o;
+  if (o != 0 && o != 8 && (o * ds2 * 4 <= 64 || wide_pt(ds2, o))) return o;
   for (int pt = 8; pt > 1; pt >>= 1) {
-    if (pt == 8 ? !pt8_ok(ds2, pad, exact) : pt * ds2 * 4 > 64) continue;
+    if (pt == 8 ? !pt8_ok(ds2, pad, exact)
+                : pt * ds2 * 4 > 64 && !wide_pt(ds2, pt))
+      continue;
     if (grid_wgs(pt, B, N) >= fill_wgs(pt, ds2, exact)) return pt;
     if (pt == 8 && K >= 8192 && grid_wgs(8, B, N) >= 2 * device_shape().cus)
       return 8;
@@ -1405,15 +1456,15 @@ static Plan plan_assign(int64_t B, int64_t N, int64_t K, int64_t D,
   // stage.
   p.whole = FKC_WHOLE_STAGE && FKC_USE_DMA && p.exact && !p.pad &&
             (p.ds2 == 1 || p.ds2 == 2 || p.ds2 == 4 || p.ds2 == 8) &&
-            K <= (p.ds2 <= 4 ? 256 : 128) &&
+            !wide_pt(p.ds2, p.pt) && K <= (p.ds2 <= 4 ? 256 : 128) &&
             grid_wgs(p.pt, B, N) <= 2 * device_shape().cus;
   if (!can_slice || p.exact) return p;
   // Four tiles, not eight: on sliced-size grids four tiles on ~256
   // workgroups beat eight on 512 (N = 8192, K = 65536: 0.150 vs 0.166 ms;
   // N = 16384, K = 32768: 0.142 vs 0.156 ms).
   int pt = p.pt;
-  if (ntiles_override() == 0) pt = p.ds2 <= 4 ? 4 : p.ds2 <= 8 ? 2 : 1;
-  const int64_t tiles = grid_wgs(pt, B, N);
+  if (ntiles_override() == 0) pt = p.ds2 <= 4 ? 4 : 2;
+  int64_t tiles = grid_wgs(pt, B, N);
   int64_t S = ksplit_override();
   if (S == 0 && pt == 4 && p.ds2 == 4) {
     // D = 97..128: as many slices as fit one round of the 167-VGPR
@@ -1442,10 +1493,22 @@ static Plan plan_assign(int64_t B, int64_t N, int64_t K, int64_t D,
     }
     if (S <= 1) return p;
   } else if (S == 0) {
-    const int64_t want = fill_wgs(pt, p.ds2, p.exact);
-    if (tiles >= want) return p;
-    S = 1;
-    while (tiles * S < want && K / (2 * S) >= FKC_SLICE_MIN_ROWS) S *= 2;
+    // (Above D = 256 one tile per wave runs one workgroup per CU; two tiles
+    // run two, and beat it wherever their grid passes fill_wgs: (16384,
+    // 8192, 320) fp16 220 -> 102 us, but (1799, 16610, 408) 75 -> 106.)
+    const int64_t cus = device_shape().cus;
+    for (;;) {
+      const int64_t want = (wide_pt(p.ds2, pt) ? 2 : 4) * cus;
+      tiles = grid_wgs(pt, B, N);
+      if (tiles >= want) return p;
+      S = 1;
+      while (tiles * S < want && K / (2 * S) >= FKC_SLICE_MIN_ROWS) S *= 2;
+      if (ntiles_override() != 0 || !wide_pt(p.ds2, pt) ||
+          tiles * S >= fill_wgs(pt, p.ds2, p.exact))
+        break;
+      pt = 1;
+    }
+    const int64_t want = (wide_pt(p.ds2, pt) ? 2 : 4) * cus;
     // Slices that still leave the chip short only pay off when the unsliced
     // grid is short too.
     if (tiles * S < want &&

@@ -147,6 +147,31 @@ def test_eight_tiles_match_oracle_and_four(monkeypatch, dtype, B, N, K):
 
 
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("B,N,K,D,nt", [
+    (1, 300, 31, 136, "4"), (1, 1000, 513, 160, "4"), (2, 777, 600, 192, "4"),
+    (1, 515, 512, 216, "4"), (1, 2000, 1000, 224, "4"), (1, 257, 64, 256, "4"),
+    (1, 700, 2049, 256, "4"), (1, 300, 1, 264, "2"), (1, 130, 700, 288, "2"),
+    (1, 129, 520, 320, "2"), (2, 500, 95, 376, "2"), (1, 385, 640, 480, "2"),
+    (1, 127, 33, 512, "2"), (2, 300, 1025, 512, "2"), (1, 300, 544, 504, "2"),
+])
+def test_wide_rows_with_more_tiles(monkeypatch, dtype, B, N, K, D, nt):
+    """Four tiles per wave above D = 128 and two above 256 against one, bit
+    for bit, and the oracle: padded and whole widths, staged through
+    registers and directly, exact index and re-score, partial stages."""
+    x, c = _data(B, N, K, D, dtype, seed=N + K + D)
+    if K > 40:
+        c[:, K - 1] = c[:, 2]
+    monkeypatch.setenv("FKC_NTILES", nt)
+    got = _gpu_assign(x, c, dtype)
+    monkeypatch.setenv("FKC_NTILES", "1")
+    assert np.array_equal(got, _gpu_assign(x, c, dtype))
+    ref = O.assign(x, c, dtype)
+    # the near-tie bar of a 256-wide row, in proportion to the width
+    nd, bad, worst = near_tie_report(x, c, dtype, got, ref, rel=2.0 ** -16 * max(1.0, D / 256))
+    assert bad == 0, worst
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
 @pytest.mark.parametrize("B,N,K,D", [
     (1, 5000, 1030, 128), (2, 3001, 2100, 128), (1, 9000, 4097, 128),
     (1, 4000, 1500, 64), (3, 2000, 1300, 64),

@@ -1413,6 +1413,25 @@ static bool use_resident(const Plan& p, int64_t B, int64_t N, int64_t K) {
          B * resident_need(pt, kResidentWaves, N) >= dev.cus;
 }
 
+// At K <= FKC_EXACT_MAX_K the exact in-loop index costs 13 vector instructions
+// per four scores against the kept scores' 8, and its loop is not pipelined;
+// it wins only on tables too short to amortise the kept scores' 128-row
+// stages and on small grids.  Same-box bf16 assign times (us), exact index
+// against kept scores with four tiles: D = 128, K = 512: N = 40000 13.0 /
+// 12.1, 65536 15.2 / 12.2, 100000 24.5 / 17.2, 131072 20.0 / 17.8, 262144
+// 43.2 / 34.1, 524288 70.6 / 61.3; K = 256: 40000 8.4 / 8.6, 65536 9.8 / 8.6,
+// 524288 43.3 / 39.0; K = 128: 200000 15.3 / 15.5; K = 64: 262144 15.1 / 17.2.
+// D = 64, K = 512: 200000 22.2 / 20.6, 1000000 73.3 / 62.3; K = 384: 262144
+// 18.5 / 18.4; K = 256: 262144 14.7 / 15.7.
+static bool keep_small(const Plan& p, int64_t B, int64_t N, int64_t K) {
+  if (p.pad || K > FKC_EXACT_MAX_K || save_override() == 0 ||
+      (ntiles_override() != 0 && ntiles_override() != 4))
+    return false;
+  const int64_t cus = device_shape().cus, wgs = grid_wgs(4, B, N);
+  if (p.ds2 == 4) return K > 128 && 4 * wgs >= 3 * cus;
+  return p.ds2 == 2 && K > 256 && wgs >= 3 * cus;
+}
+
 // Launch plan.  K is sliced only when no unsliced grid fills the chip (few
 // points, many centroids): the most tiles the point budget allows (four up
 // to D = 128) then run on S slices of kspan rows
@@ -1442,6 +1461,12 @@ static Plan plan_assign(int64_t B, int64_t N, int64_t K, int64_t D,
   p.pt = choose_pt(p.ds2, p.pad, p.exact, B, N, K);
   p.S = 1;
   p.kspan = (int)K;
+  if (resident_override() != 1 && keep_small(p, B, N, K)) {
+    p.exact = false;
+    p.save = true;
+    p.pt = 4;
+    return p;
+  }
   if (use_resident(p, B, N, K)) {
     p.resident = true;
     p.exact = false;

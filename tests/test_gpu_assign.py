@@ -200,6 +200,29 @@ def test_saved_scores_match_rescore(monkeypatch, dtype, B, N, K, D):
         _check(x, c, dtype, outs[0], max_frac=1e-3)
 
 
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("B,N,K,D", [
+    (1, 49153, 129, 128), (1, 65536, 256, 128), (3, 20001, 383, 128), (1, 50000, 512, 128),
+    (1, 196609, 257, 64), (2, 100001, 511, 64),
+])
+def test_kept_scores_at_small_k(monkeypatch, dtype, B, N, K, D):
+    """Grids that keep the winning block's scores although K is within the
+    exact-index cutoff, against the exact index bit for bit (FKC_SAVE=0):
+    equal rows, infinities and NaN rows among the points and centroids."""
+    x, c = _data(B, N, K, D, "f32", seed=N + K)
+    c[:, K - 1] = c[:, 3]
+    c[:, 17] = c[:, 16]
+    c[:, K // 2, 5] = np.inf
+    x[:, 5] = np.nan
+    x[:, 6, 0] = -np.inf
+    x[:, 7, 1] = np.nan
+    x, c = O.from_f32(x, dtype), O.from_f32(c, dtype)
+    got = _gpu_assign(x, c, dtype)
+    monkeypatch.setenv("FKC_SAVE", "0")
+    assert np.array_equal(got, _gpu_assign(x, c, dtype))
+    assert not np.isin(got, [K - 1, 17]).any()
+
+
 RESIDENT_CASES = [
     # (B, N, K, D): one centroid, K below and not a multiple of 16, ragged N,
     # batches, c4's shape at reduced N, and the largest tables that fit one

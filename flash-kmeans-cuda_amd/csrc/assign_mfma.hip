@@ -1424,12 +1424,13 @@ static bool use_resident(const Plan& p, int64_t B, int64_t N, int64_t K) {
 // D = 64, K = 512: 200000 22.2 / 20.6, 1000000 73.3 / 62.3; K = 384: 262144
 // 18.5 / 18.4; K = 256: 262144 14.7 / 15.7.
 static bool keep_small(const Plan& p, int64_t B, int64_t N, int64_t K) {
-  if (p.pad || K > FKC_EXACT_MAX_K || save_override() == 0 ||
-      (ntiles_override() != 0 && ntiles_override() != 4))
+  if (p.pad || K > FKC_EXACT_MAX_K || K <= (p.ds2 == 4 ? 128 : 256) ||
+      (p.ds2 != 4 && p.ds2 != 2))
     return false;
   const int64_t cus = device_shape().cus, wgs = grid_wgs(4, B, N);
-  if (p.ds2 == 4) return K > 128 && 4 * wgs >= 3 * cus;
-  return p.ds2 == 2 && K > 256 && wgs >= 3 * cus;
+  if (p.ds2 == 4 ? 4 * wgs < 3 * cus : wgs < 3 * cus) return false;
+  const int nt = ntiles_override();
+  return (nt == 0 || nt == 4) && save_override() != 0 && resident_override() != 1;
 }
 
 // Launch plan.  K is sliced only when no unsliced grid fills the chip (few
@@ -1443,7 +1444,7 @@ static bool keep_small(const Plan& p, int64_t B, int64_t N, int64_t K) {
 // took 0.376 ms against 0.756 ms, and at N = 8192, K = 65536, D = 128
 // eight slices 0.150 ms against 0.531 ms.  At D = 97..128 the slices fill
 // one round of resident workgroups (below).  FKC_KSPLIT forces S.
-static Plan plan_assign(int64_t B, int64_t N, int64_t K, int64_t D,
+static Plan plan_filled(int64_t B, int64_t N, int64_t K, int64_t D,
                         bool can_slice) {
   Plan p;
   p.ds2 = (int)((D + 31) / 32);
@@ -1461,7 +1462,7 @@ static Plan plan_assign(int64_t B, int64_t N, int64_t K, int64_t D,
   p.pt = choose_pt(p.ds2, p.pad, p.exact, B, N, K);
   p.S = 1;
   p.kspan = (int)K;
-  if (resident_override() != 1 && keep_small(p, B, N, K)) {
+  if (keep_small(p, B, N, K)) {
     p.exact = false;
     p.save = true;
     p.pt = 4;
@@ -1550,6 +1551,73 @@ static Plan plan_assign(int64_t B, int64_t N, int64_t K, int64_t D,
   return p;
 }
 
+// Calls of fewer points keep the slice counts of plan_filled, by which their
+// callers' small workspaces have always been sized.
+constexpr int64_t kShortSliceMinPoints = 1000;
+
+// Modelled time (us, without the launch) of w workgroups per CU that score
+// kspan rows each: a lone wave's 16-row block takes its fragment reads (42
+// cycles per 32 features) and its MFMAs in turn, several share the matrix
+// pipe (19 cycles per tile and 32 features, stalls included) or the LDS (34);
+// a workgroup's start and end cost 2.5 us with kept scores and 3 + 0.7 per 32
+// features with the re-score; merging S slices 3 + 0.03 S.  Fitted to fp16
+// launches of 1000 .. 32768 points.
+static double grid_model(const Plan& p, int64_t wgs, int64_t cus) {
+  const int64_t w = (wgs + cus - 1) / cus;
+  const double cycles = std::max(42.0 + 16.0 * p.pt,
+                                 (double)w * std::max(19.0 * p.pt, 34.0));
+  return (double)((p.kspan + 15) / 16) * p.ds2 * cycles * 0.476e-3 +
+         (double)w * (p.save ? 2.5 : 3.0 + 0.7 * p.ds2) +
+         (p.S > 1 ? 3.0 + 0.03 * p.S : 0.0);
+}
+
+// Grids that leave CUs idle although they may slice (few points, a K below
+// what FKC_SLICE_MIN_ROWS-row slices need to fill them): the tiles per wave
+// and the slice count, down to 128 rows, with the least modelled time.  Only
+// where the launch is modelled at 17 us or more, so that the merge's launch is
+// repaid also where the host is busy enqueueing, and the gain at
+// 22%.  Same-box fp16 (us, before and after): (1000, 4096, 128) 34 / 13,
+// (4096, 4096, 128) 34 / 13, (8192, 2048, 128) 22 / 12, (32768, 2048, 128)
+// 28 / 21, (4096, 8192, 64) 27 / 13, (1000, 2048, 256) 36 / 14, (8192, 4096,
+// 256) 50 / 34; labels are the same for every slicing.
+static Plan plan_assign(int64_t B, int64_t N, int64_t K, int64_t D,
+                        bool can_slice) {
+  const Plan p = plan_filled(B, N, K, D, can_slice);
+  if (!can_slice || p.exact || p.resident || K <= FKC_EXACT_MAX_K ||
+      B * N < kShortSliceMinPoints)
+    return p;
+  const int64_t cus = device_shape().cus;
+  const int64_t old_wgs = grid_wgs(p.pt, B, N) * p.S;
+  const double old = grid_model(p, old_wgs, cus);
+  if (old_wgs >= 2 * cus || old < 17.0 || ksplit_override() != 0 ||
+      ntiles_override() != 0)
+    return p;
+  Plan best = p;
+  double least = 0.78 * old;
+  for (int pt = 4; pt >= 1; pt >>= 1) {
+    if (pt * p.ds2 * 4 > 64) continue;
+    const int64_t tiles = grid_wgs(pt, B, N);
+    for (int64_t per = 1; per <= 3; ++per) {  // workgroups per CU
+      const int64_t want = std::min<int64_t>(per * cus / tiles, K / 128);
+      if (want < 2) continue;
+      const int64_t span = ((K + want - 1) / want + 127) / 128 * 128;
+      const int64_t S = (K + span - 1) / span;
+      if (S <= 1) continue;
+      Plan q = p;
+      q.pt = pt;
+      q.S = (int)S;
+      q.kspan = (int)span;
+      q.save = use_save(q, tiles * S);
+      const double t = grid_model(q, tiles * S, cus);
+      if (t < least) {
+        least = t;
+        best = q;
+      }
+    }
+  }
+  return best;
+}
+
 static size_t slice_bytes(const Plan& p, int64_t B, int64_t N, Slices* sl,
                           void* ws) {
   if (p.S <= 1) return 0;
@@ -1566,9 +1634,11 @@ static size_t slice_bytes(const Plan& p, int64_t B, int64_t N, Slices* sl,
 }
 
 size_t assign_workspace_bytes(int64_t B, int64_t N, int64_t K, int64_t D,
-                              int dtype) {
+                              int dtype, bool least) {
   if (!assign_uses_mfma(dtype, D) || B * N == 0 || K < 1) return 0;
-  return slice_bytes(plan_assign(B, N, K, D, true), B, N, nullptr, nullptr);
+  return slice_bytes(least ? plan_filled(B, N, K, D, true)
+                           : plan_assign(B, N, K, D, true),
+                     B, N, nullptr, nullptr);
 }
 
 int launch_assign_mfma(const void* x, const void* c, const float* c_sq,

@@ -65,8 +65,8 @@ int fkc_kmeans_lloyd_noalloc(const void* x, const void* init_centroids,
                              int64_t N, int64_t K, int64_t D, int dtype,
                              int max_iters, float tol, fkc_stream_t stream,
                              int32_t* n_iters_dev, int32_t* n_iters_host) {
-  const size_t need =
-      fkc_kmeans_workspace_bytes(B, N, K, D, dtype, max_iters < 0 ? 0 : max_iters);
+  const size_t need = fkc::lloyd_least_workspace_bytes(
+      B, N, K, D, dtype, max_iters < 0 ? 0 : max_iters);
   if (need > fkc::kScratchBytes)
     return fkc::fail(FKC_ERR_WORKSPACE,
                      "kmeans_lloyd_noalloc: this shape needs %zu bytes of "
@@ -76,7 +76,8 @@ int fkc_kmeans_lloyd_noalloc(const void* x, const void* init_centroids,
   if (int rc = fkc::scratch_on_current_device(&ws)) return rc;
   return fkc::lloyd_run(x, init_centroids, centroids, cluster_ids, B, N, K, D,
                         dtype, max_iters, tol, ws, fkc::kScratchBytes, stream,
-                        n_iters_dev, n_iters_host, /*profile=*/false);
+                        n_iters_dev, n_iters_host, /*profile=*/false,
+                        /*fixed_ws=*/true);
 }
 
 }  // extern "C"

@@ -42,8 +42,10 @@ struct Carve {
 bool assign_uses_mfma(int dtype, int64_t D);
 // Workspace bytes of a sliced MFMA assign (centroid slices scored by
 // separate workgroups, then merged) for this shape; 0 when it is not sliced.
+// least: without the slices that only shorten underfilled launches (what a
+// caller with a workspace of fixed size judges a shape by).
 size_t assign_workspace_bytes(int64_t B, int64_t N, int64_t K, int64_t D,
-                              int dtype);
+                              int dtype, bool least = false);
 // ev0 / ev1 (optional, both or neither): timing events of the launch; on
 // the MFMA route the dispatch packets stamp them (no extra stream packets).
 // ws (optional, assign_workspace_bytes): with it the MFMA route may slice K;
@@ -210,12 +212,17 @@ int launch_sampled_inertia(const void* x, const void* c, const int32_t* idx,
 
 // ---------------------------------------------------------------- loop
 // The Lloyd loop behind fkc_kmeans_lloyd*; profile = false ignores the
-// profiling hook (creates no events).
+// profiling hook (creates no events); fixed_ws: a workspace too small for
+// the assign's slices runs it unsliced instead of being refused.
 int lloyd_run(const void* x, const void* init, void* centroids,
               int32_t* cluster_ids, int64_t B, int64_t N, int64_t K,
               int64_t D, int dtype, int max_iters, float tol, void* workspace,
               size_t workspace_bytes, fkc_stream_t stream,
-              int32_t* n_iters_dev, int32_t* n_iters_host, bool profile);
+              int32_t* n_iters_dev, int32_t* n_iters_host, bool profile,
+              bool fixed_ws = false);
+// The loop's workspace with assign_workspace_bytes(..., least).
+size_t lloyd_least_workspace_bytes(int64_t B, int64_t N, int64_t K, int64_t D,
+                                 int dtype, int max_iters);
 
 // ---------------------------------------------------------------- device
 // Compute units and the LDS one workgroup may hold on the current device,

@@ -252,7 +252,8 @@ FKC_CAPI int fkc_kmeans_lloyd_from(const void* x, const void* init_centroids,
  * that forbid hipMalloc).  The loop's workspace is a static device array of
  * fkc_kmeans_noalloc_max_bytes() bytes (64 MiB) that each GPU using the
  * library holds until the process ends; a shape whose workspace
- * (fkc_kmeans_workspace_bytes) is larger is refused with FKC_ERR_WORKSPACE.
+ * (fkc_kmeans_workspace_bytes, less what slicing K only for speed adds: such
+ * slices are given up first) is larger is refused with FKC_ERR_WORKSPACE.
  * The array is looked up once per device, on the first call made with that
  * device current; stream must belong to the current device.  Every call on
  * one GPU shares the array: calls that overlap on one GPU (other streams or

@@ -302,6 +302,28 @@ def test_sliced_assign_matches_unsliced(monkeypatch, B, N, K, D, dtype, ksplit):
     _check(x, c, dtype, got, max_frac=1e-3)
 
 
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("B,N,K,D", [
+    (1, 1000, 2048, 128), (60, 17, 2500, 128), (2, 3001, 3900, 64), (1, 5000, 4100, 32),
+    (1, 4097, 1500, 200), (1, 1025, 1025, 256), (4, 300, 2000, 512), (3, 999, 3000, 96),
+])
+def test_underfilled_grids_slice_k(monkeypatch, dtype, B, N, K, D):
+    """Few points and a K below the whole-slice rule: short slices (down to
+    128 rows, with kept scores or the re-score) against the unsliced launch,
+    bit for bit, with equal rows in different slices."""
+    from flash_kmeans_cuda import _lib
+    monkeypatch.delenv("FKC_KSPLIT", raising=False)
+    x, c = _data(B, N, K, D, dtype, seed=N + K + D)
+    c[:, K - 1] = c[:, 7]
+    c[:, K // 2] = c[:, 8]
+    dt = {"f16": 1, "bf16": 2}[dtype]
+    assert _lib.lib.fkc_euclid_assign_workspace_bytes(B, N, K, D, dt) > 0
+    got = _gpu_assign(x, c, dtype)
+    monkeypatch.setenv("FKC_KSPLIT", "1")
+    assert np.array_equal(got, _gpu_assign(x, c, dtype))
+    assert not np.isin(got, [K - 1, K // 2]).any()
+
+
 def test_sliced_assign_workspace_errors(monkeypatch):
     """fkc_euclid_assign_ws rejects a short or misaligned workspace with
     FKC_ERR_WORKSPACE before launching anything, and needs none when the

@@ -91,6 +91,30 @@ def test_no_alloc_refuses_shapes_beyond_the_scratch():
     assert rc == 2 and "static scratch" in _lib.last_error()
 
 
+def test_no_alloc_gives_up_slices_before_it_refuses(monkeypatch):
+    """A shape that fits the static scratch without the slices of an
+    underfilled assign, but not with them, still runs, with the same bits."""
+    from flash_kmeans_cuda import _lib
+    cap = _lib.lib.fkc_kmeans_noalloc_max_bytes()
+    B, N, D = 8, 130, 512
+
+    def need(K, split):
+        if split:
+            monkeypatch.setenv("FKC_KSPLIT", split)
+        else:
+            monkeypatch.delenv("FKC_KSPLIT", raising=False)
+        return _lib.lib.fkc_kmeans_workspace_bytes(B, N, K, D, 1, 2)
+
+    K = next(k for k in range(4095, 3000, -1) if need(k, "1") <= cap)
+    assert need(K, None) > cap  # (whole slices would need K >= 4096)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    x = torch.randn(B, N, D, device="cuda", generator=g).half()
+    init = torch.randn(B, K, D, device="cuda", generator=g).half()
+    a = _with_workspace(x, init, K, 2, 0.0)
+    b = _no_alloc(x, init, K, 2, 0.0)
+    assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
+
+
 _CAPTURED_NO_ALLOC = r'''
 import sys, torch
 sys.path.insert(0, sys.argv[1])

@@ -16,8 +16,7 @@
 //                    lane accumulates its squares in fp64 in row order; the
 //                    wave and then the workgroup combine lanes in a fixed
 //                    order into one partial per workgroup.  Lane r of the
-//                    wave also counts row r's label into the K-bin histogram
-//                    (integer atomics: exact).
+//                    wave also marks row r's label in the K-bin table.
 //   quality_final  : one workgroup per batch row sums the partials in a
 //                    fixed order; workgroup 0 also counts the empty bins.
 //   sample_gather  : the sampled rows of x, for the sampled inertia
@@ -41,7 +40,14 @@ __device__ inline double wave_sum_f64(double v) {
   return v;
 }
 
-template <int DT>
+// NI: 64-column slices of a row (D <= 64 NI), or 0 for any D, one row at a
+// time.  With NI known the rows are loaded in batches (64 elements of x and
+// 64 of the centroids in flight per lane) and accumulated in row order, the
+// same sums: one row at a time left the kernel waiting for a round trip per
+// row ((1, 262144, 4096, 128) fp16 62 us, and 40 us for 4096 sampled rows on
+// 16 workgroups).  Bound by the loads: 2 D bytes of x per row from HBM and as
+// many of its centroid from the caches.
+template <int DT, int NI>
 __global__ void __launch_bounds__(QT)
 quality_rows_kernel(const typename Elem<DT>::T* __restrict__ x,
                     const typename Elem<DT>::T* __restrict__ cent,
@@ -50,6 +56,7 @@ quality_rows_kernel(const typename Elem<DT>::T* __restrict__ x,
                     int N, int K, int D, int nwg,
                     const int32_t* __restrict__ sidx, int sN) {
   using E = Elem<DT>;
+  using T = typename E::T;
   __shared__ double wsum[QT / 64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int b = blockIdx.y;
@@ -60,22 +67,57 @@ quality_rows_kernel(const typename Elem<DT>::T* __restrict__ x,
   // counts as unlabelled.
   const bool sok = sidx == nullptr || (my < N && (uint32_t)sidx[my] < (uint32_t)sN);
   const int iv = my < N && sok ? ib[my] : -1;
-  if (hist != nullptr && (uint32_t)iv < (uint32_t)K) atomicAdd(&hist[iv], 1);
+  // Only zero or not is read: every writer stores the same 1.
+  if (hist != nullptr && (uint32_t)iv < (uint32_t)K) hist[iv] = 1;
 
   double acc = 0.0;
   if (x != nullptr) {
-    const typename E::T* xb = x + (size_t)b * N * D;
-    const typename E::T* cb = cent + (size_t)b * K * D;
+    const T* xb = x + (size_t)b * N * D;
+    const T* cb = cent + (size_t)b * K * D;
     const int nr = min(QROWS, N - r0);
-    for (int j = 0; j < nr; ++j) {
-      const int id = __builtin_amdgcn_readlane(iv, j);
-      if ((uint32_t)id >= (uint32_t)K) continue;  // wave-uniform
-      const typename E::T* xr = xb + (size_t)(r0 + j) * D;
-      const typename E::T* cr = cb + (size_t)id * D;
-      for (int d = lane; d < D; d += 64) {
-        const float df = E::load(xr[d]) - E::load(cr[d]);
-        const float sq = df * df;  // fp32 square, as the reference
-        acc += (double)sq;
+    if constexpr (NI == 0) {
+      for (int j = 0; j < nr; ++j) {
+        const int id = __builtin_amdgcn_readlane(iv, j);
+        if ((uint32_t)id >= (uint32_t)K) continue;  // wave-uniform
+        const T* xr = xb + (size_t)(r0 + j) * D;
+        const T* cr = cb + (size_t)id * D;
+        for (int d = lane; d < D; d += 64) {
+          const float df = E::load(xr[d]) - E::load(cr[d]);
+          const float sq = df * df;  // fp32 square, as the reference
+          acc += (double)sq;
+        }
+      }
+    } else {
+      constexpr int RB = 64 / NI < 16 ? 64 / NI : 16;  // rows in flight
+      int col[NI];
+#pragma unroll
+      for (int i = 0; i < NI; ++i) col[i] = min(lane + 64 * i, D - 1);
+      for (int j0 = 0; j0 < nr; j0 += RB) {
+        T xv[RB][NI], cv[RB][NI];
+#pragma unroll
+        for (int j = 0; j < RB; ++j) {
+          // Rows past the wave's last, and rows of no cluster, load rows
+          // that exist and are not accumulated.
+          const int id = __builtin_amdgcn_readlane(iv, j0 + j);
+          const T* xr = xb + (size_t)min(r0 + j0 + j, N - 1) * D;
+          const T* cr = cb + (size_t)((uint32_t)id < (uint32_t)K ? id : 0) * D;
+#pragma unroll
+          for (int i = 0; i < NI; ++i) {
+            xv[j][i] = xr[col[i]];
+            cv[j][i] = cr[col[i]];
+          }
+        }
+#pragma unroll
+        for (int j = 0; j < RB; ++j) {
+          const int id = __builtin_amdgcn_readlane(iv, j0 + j);
+          if ((uint32_t)id >= (uint32_t)K) continue;  // past N: -1
+#pragma unroll
+          for (int i = 0; i < NI; ++i) {
+            const float df = E::load(xv[j][i]) - E::load(cv[j][i]);
+            const float sq = df * df;  // fp32 square, as the reference
+            acc += lane + 64 * i < D ? (double)sq : 0.0;
+          }
+        }
       }
     }
   }
@@ -147,11 +189,18 @@ int launch_rows_t(const void* x, const void* c, const int32_t* ids,
                   int64_t K, int64_t D, int64_t nwg, const int32_t* sidx,
                   int64_t sN, hipStream_t s) {
   using T = typename Elem<DT>::T;
-  hipLaunchKernelGGL((quality_rows_kernel<DT>), dim3((unsigned)nwg, (unsigned)B),
-                     dim3(QT), 0, s, static_cast<const T*>(x),
-                     static_cast<const T*>(c), ids, partial, hist, (int)N,
-                     (int)K, (int)D, (int)nwg, sidx, (int)sN);
-  return check_launch("quality_rows");
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)nwg, (unsigned)B), dim3(QT), 0, s,
+                       static_cast<const T*>(x), static_cast<const T*>(c), ids,
+                       partial, hist, (int)N, (int)K, (int)D, (int)nwg, sidx,
+                       (int)sN);
+    return check_launch("quality_rows");
+  };
+  if (D <= 64) return go(quality_rows_kernel<DT, 1>);
+  if (D <= 128) return go(quality_rows_kernel<DT, 2>);
+  if (D <= 256) return go(quality_rows_kernel<DT, 4>);
+  if (D <= 512) return go(quality_rows_kernel<DT, 8>);
+  return go(quality_rows_kernel<DT, 0>);
 }
 
 }  // namespace
@@ -171,6 +220,7 @@ size_t sample_workspace_bytes(int64_t B, int64_t S, int64_t K, int64_t D,
   c.take<float>((size_t)B * S);                         // their x_sq
   c.take<float>((size_t)B * K);                         // c_sq
   c.take<int32_t>((size_t)B * S);                       // their labels
+  c.take<char>(assign_workspace_bytes(B, S, K, D, dtype));
   c.take<char>(quality_workspace_bytes(B, S, K));
   return c.used;
 }
@@ -192,6 +242,8 @@ int launch_sampled_inertia(const void* x, const void* c, const int32_t* idx,
   float* xs_sq = cv.take<float>((size_t)B * S);
   float* c_sq = cv.take<float>((size_t)B * K);
   int32_t* lab = cv.take<int32_t>((size_t)B * S);
+  const size_t abytes = assign_workspace_bytes(B, S, K, D, dtype);
+  void* aws = abytes ? cv.take<char>(abytes) : nullptr;
   const size_t qbytes = quality_workspace_bytes(B, S, K);
   void* qws = cv.take<char>(qbytes);
   const int row_bytes = (int)(D * dtype_size(dtype));
@@ -204,7 +256,8 @@ int launch_sampled_inertia(const void* x, const void* c, const int32_t* idx,
   if (!rc && !assign_uses_mfma(dtype, D))
     rc = launch_row_sqnorm(xs, xs_sq, B * S, D, dtype, nullptr, s);
   if (!rc)
-    rc = launch_assign(xs, c, xs_sq, c_sq, lab, B, S, K, D, dtype, nullptr, s);
+    rc = launch_assign(xs, c, xs_sq, c_sq, lab, B, S, K, D, dtype, nullptr, s,
+                       nullptr, nullptr, aws, abytes);
   if (!rc)
     rc = launch_quality(xs, c, lab, B, S, K, D, dtype, inertia, nullptr, qws,
                         qbytes, s, idx, N);

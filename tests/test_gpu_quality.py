@@ -67,6 +67,21 @@ def test_inertia_and_empty_match_oracle(B, N, K, D, dtype):
     assert got_e == want_e
 
 
+@pytest.mark.parametrize("D", [1, 63, 64, 65, 128, 129, 255, 256, 257, 511, 512, 513])
+@pytest.mark.parametrize("N,dtype", [(1, "f32"), (63, "f16"), (257, "bf16"), (1000, "f32")])
+def test_inertia_over_row_batches(D, N, dtype):
+    """Rows in flight: every column-slice count, the last rows of a wave and
+    of a workgroup, labels outside [0, K) inside a batch."""
+    rng = np.random.default_rng(D * 7 + N)
+    x = O.from_f32(rng.standard_normal((2, N, D)).astype(np.float32) * 2, dtype)
+    c = O.from_f32(rng.standard_normal((2, 9, D)).astype(np.float32) * 2, dtype)
+    ids = rng.integers(-1, 11, (2, N)).astype(np.int32)
+    ids[0, 0] = 4
+    got_i, got_e = _device(x, ids, c, dtype)
+    assert np.allclose(got_i, O.assigned_inertia(x, ids, c, dtype), rtol=1e-10, atol=0)
+    assert got_e == O.empty_clusters(ids, 9)
+
+
 def test_bitwise_reproducible():
     rng = np.random.default_rng(3)
     x = O.from_f32(rng.standard_normal((1, 300000, 128)).astype(np.float32), "f16")

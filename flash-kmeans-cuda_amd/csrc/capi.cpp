@@ -250,6 +250,27 @@ LoopBuffers carve_loop(void* ws, int64_t B, int64_t N, int64_t K, int64_t D,
   if (total) *total = c.used;
   return L;
 }
+struct UpdateBuffers {
+  int32_t* sorted = nullptr;
+  int32_t* perm = nullptr;
+  void* sort_ws = nullptr;
+  size_t sort_ws_bytes = 0;
+  void* upd_ws = nullptr;
+  size_t upd_ws_bytes = 0;
+};
+UpdateBuffers carve_centroid_update(void* ws, int64_t B, int64_t N, int64_t K,
+                                    int64_t D, size_t* total) {
+  Carve c(ws);
+  UpdateBuffers u;
+  u.sorted = c.take<int32_t>((size_t)B * N);
+  u.perm = c.take<int32_t>((size_t)B * N);
+  u.sort_ws_bytes = sort_workspace_bytes(B, N, K);
+  u.sort_ws = c.take<char>(u.sort_ws_bytes);
+  u.upd_ws_bytes = update_workspace_bytes(B, N, D);
+  u.upd_ws = c.take<char>(u.upd_ws_bytes);
+  if (total) *total = c.used;
+  return u;
+}
 }  // namespace
 }  // namespace fkc
 
@@ -385,6 +406,53 @@ int fkc_centroid_update_sorted_indexed(const void* x, const int32_t* sorted_idx,
   return update_common(x, sorted_idx, ids_sorted, sums, counts, B, N, K, D,
                        dtype, workspace, workspace_bytes, stream,
                        "centroid_update_sorted_indexed");
+}
+
+size_t fkc_centroid_update_workspace_bytes(int64_t B, int64_t N, int64_t K,
+                                           int64_t D) {
+  if (B <= 0 || N <= 0 || K < 1 || D < 1) return 0;
+  size_t total = 0;
+  carve_centroid_update(nullptr, B, N, K, D, &total);
+  return total;
+}
+
+// The sort's control region, the sums and the counts are cleared by one
+// launch: at (4, 131072, 512, 128) bf16 three launches of 4.5 to 4.8 us.
+int fkc_centroid_update(const void* x, const int32_t* cluster_ids, float* sums,
+                        int32_t* counts, int64_t B, int64_t N, int64_t K,
+                        int64_t D, int dtype, void* workspace,
+                        size_t workspace_bytes, fkc_stream_t stream) {
+  g_err[0] = 0;
+  if (int rc = shape_ok(B, N, K, D, "centroid_update")) return rc;
+  if (int rc = dtype_ok(dtype, "centroid_update")) return rc;
+  if (B == 0) return FKC_OK;
+  if (!sums || !counts || (N > 0 && (!x || !cluster_ids)))
+    return fail(FKC_ERR_INVALID, "centroid_update: null pointer argument");
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  ZeroFill zf;
+  zf.z2 = sums;
+  zf.n2 = B * K * D;
+  zf.z3 = counts;
+  zf.n3 = B * K;
+  if (N == 0) return launch_zero(zf, s);
+  const size_t need = fkc_centroid_update_workspace_bytes(B, N, K, D);
+  if (!workspace || workspace_bytes < need)
+    return fail(FKC_ERR_WORKSPACE, "centroid_update: workspace %zu < %zu bytes",
+                workspace_bytes, need);
+  if (reinterpret_cast<uintptr_t>(workspace) % kWorkspaceAlign != 0)
+    return fail(FKC_ERR_WORKSPACE,
+                "centroid_update: workspace not %d-byte aligned",
+                kWorkspaceAlign);
+  const UpdateBuffers u = carve_centroid_update(workspace, B, N, K, D, nullptr);
+  label_sort_reset_region(u.sort_ws, B, N, K, &zf.z0, &zf.n0);
+  int rc = launch_zero(zf, s);
+  if (!rc)
+    rc = launch_label_sort(cluster_ids, u.sorted, u.perm, B, N, K, false,
+                           u.sort_ws, u.sort_ws_bytes, nullptr, s, 0);
+  if (!rc)
+    rc = launch_update(x, u.perm, u.sorted, sums, counts, B, N, K, D, dtype,
+                       false, u.upd_ws, u.upd_ws_bytes, nullptr, s);
+  return rc;
 }
 
 int fkc_centroid_finalize(const float* sums, const int32_t* counts,

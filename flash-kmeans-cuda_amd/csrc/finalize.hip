@@ -73,6 +73,21 @@ __global__ void fill_f32_kernel(float* p, float v, int64_t n) {
   for (int64_t j = i; j < n; j += stride) p[j] = v;
 }
 
+// Several regions cleared in one launch (the loop's prologue does the same
+// beside its rows).
+__global__ void __launch_bounds__(256)
+zero_regions_kernel(int32_t* __restrict__ z0, int64_t n0,
+                    int32_t* __restrict__ z1, int64_t n1,
+                    float* __restrict__ z2, int64_t n2,
+                    int32_t* __restrict__ z3, int64_t n3) {
+  const int64_t i0 = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t stride = (int64_t)gridDim.x * 256;
+  for (int64_t i = i0; i < n0; i += stride) z0[i] = 0;
+  for (int64_t i = i0; i < n1; i += stride) z1[i] = 0;
+  for (int64_t i = i0; i < n2; i += stride) z2[i] = 0.f;
+  for (int64_t i = i0; i < n3; i += stride) z3[i] = 0;
+}
+
 __global__ void fill_f64_kernel(double* p, double v, int64_t n) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
@@ -229,6 +244,16 @@ int launch_fill_i32(int32_t* p, int32_t v, int64_t n, hipStream_t s) {
   hipLaunchKernelGGL(fill_i32_kernel, dim3(grid_for(n)), dim3(256), 0, s, p, v,
                      n);
   return check_launch("fill_i32");
+}
+
+int launch_zero(const ZeroFill& f, hipStream_t s) {
+  int64_t n = f.n0 > f.n1 ? f.n0 : f.n1;
+  n = n > f.n2 ? n : f.n2;
+  n = n > f.n3 ? n : f.n3;
+  if (n <= 0) return FKC_OK;
+  hipLaunchKernelGGL(zero_regions_kernel, dim3(grid_for(n)), dim3(256), 0, s,
+                     f.z0, f.n0, f.z1, f.n1, f.z2, f.n2, f.z3, f.n3);
+  return check_launch("zero_regions");
 }
 
 int launch_fill_f32(float* p, float v, int64_t n, hipStream_t s) {

@@ -175,6 +175,8 @@ struct ZeroFill {
   int32_t* z3 = nullptr;
   int64_t n3 = 0;
 };
+// The zero-fills alone, in one launch.
+int launch_zero(const ZeroFill& f, hipStream_t s);
 // One launch: cent = init (when the pointers differ), c_sq = row squared
 // norms of init (the bits of launch_row_sqnorm), and the zero-fills.
 int launch_lloyd_prologue(const void* init, void* cent, float* c_sq,

@@ -39,6 +39,8 @@ SIGNATURES = {
     "fkc_update_workspace_bytes": (_sz, [_i64, _i64, _i64]),
     "fkc_centroid_update_sorted": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _vp, _sz, _vp]),
     "fkc_centroid_update_sorted_indexed": (_int, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _vp, _sz, _vp]),
+    "fkc_centroid_update_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64]),
+    "fkc_centroid_update": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _vp, _sz, _vp]),
     "fkc_centroid_finalize": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _int, _vp]),
     "fkc_kmeans_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64, _int, _int]),
     "fkc_kmeans_lloyd": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _int, ctypes.c_float, _vp, _sz, _vp, _vp, _vp]),

@@ -118,12 +118,20 @@ def centroid_update_sorted(
     x = _gpu_dense("x", x)
     cluster_ids = _as_i32(_gpu_dense("cluster_ids", cluster_ids))
     B, N, D = x.shape
-    sorted_ids, perm = label_sort(cluster_ids, K)
-    sums = (torch.zeros((B, K, D), device=x.device, dtype=torch.float32)
-            if sums_out is None else sums_out.zero_())
-    counts = (torch.zeros((B, K), device=x.device, dtype=torch.int32)
-              if counts_out is None else counts_out.zero_())
-    _C.centroid_update_sorted_indexed(x, perm, sorted_ids, sums, counts)
+    sums = (torch.empty((B, K, D), device=x.device, dtype=torch.float32)
+            if sums_out is None else sums_out)
+    counts = (torch.empty((B, K), device=x.device, dtype=torch.int32)
+              if counts_out is None else counts_out)
+    if _C._check_update(x, cluster_ids, sums, counts, "centroid_update_sorted")[2] != K:
+        # A buffer of another K: labels up to its own K count, in any order.
+        sorted_ids, perm = label_sort(cluster_ids, K)
+        _C.centroid_update_sorted_indexed(x, perm, sorted_ids, sums.zero_(), counts.zero_())
+        return sums, counts
+    ws = _lib.workspace(_lib.lib.fkc_centroid_update_workspace_bytes(B, N, K, D), x.device)
+    _lib.check(_lib.lib.fkc_centroid_update(
+        x.data_ptr(), cluster_ids.data_ptr(), sums.data_ptr(), counts.data_ptr(), B, N, K, D,
+        _lib.dtype_code(x.dtype), ws.data_ptr(), ws.numel(), _lib.stream_of(x)),
+        "centroid_update_sorted")
     return sums, counts
 
 

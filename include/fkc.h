@@ -154,6 +154,20 @@ FKC_CAPI int fkc_centroid_update_sorted_indexed(
     int dtype, void* workspace, size_t workspace_bytes, fkc_stream_t stream);
 
 /*
+ * Sums and counts of labels in any order, in one call: clears sums (B,K,D)
+ * and counts (B,K), sorts the labels (fkc_label_sort) and adds the rows
+ * (fkc_centroid_update_sorted_indexed), with the bits of those calls.
+ * Replaces ops.centroid_update_sorted (flash_kmeans_cuda/ops.py:58-112).
+ */
+FKC_CAPI size_t fkc_centroid_update_workspace_bytes(int64_t B, int64_t N,
+                                                    int64_t K, int64_t D);
+FKC_CAPI int fkc_centroid_update(const void* x, const int32_t* cluster_ids,
+                                 float* sums, int32_t* counts, int64_t B,
+                                 int64_t N, int64_t K, int64_t D, int dtype,
+                                 void* workspace, size_t workspace_bytes,
+                                 fkc_stream_t stream);
+
+/*
  * out[b,k,:] = counts[b,k] > 0 ? cast(sums[b,k,:] / counts[b,k]) : old[b,k,:]
  * (IEEE division, round-to-nearest-even cast).  out may alias old.
  * Replaces fkc::centroid_finalize_out (flash_kmeans_cuda.h:71-75) and

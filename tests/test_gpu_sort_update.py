@@ -330,3 +330,35 @@ def test_update_unsorted_labels(K, D, dtype):
     assert np.array_equal(c, ec)
     tol = 1e-6 * np.maximum(ec[..., None], 1) * np.abs(O.to_f64(x, dtype)).max()
     assert np.all(np.abs(s - es) <= tol + 1e-5)
+
+
+@pytest.mark.parametrize("B,N,K,D,dtype", [
+    (1, 1, 1, 1, "f32"), (1, 300, 7, 3, "f16"), (2, 4097, 300, 128, "bf16"),
+    (3, 1000, 40, 513, "f32"), (1, 70000, 9000, 64, "f16"), (4, 9000, 2, 96, "bf16"),
+])
+def test_one_call_update_matches_the_separate_calls(B, N, K, D, dtype):
+    """fkc_centroid_update (one launch clears the sort's state, the sums and
+    the counts) against label_sort + centroid_update_sorted_indexed on
+    zeroed buffers, bit for bit: used buffers, labels outside [0, K), long
+    runs of one label, and an out buffer of another K."""
+    from flash_kmeans_cuda import _C, centroid_update_sorted
+    from flash_kmeans_cuda.ops import label_sort
+    rng = np.random.default_rng(N + K + D)
+    x = _t(O.from_f32(rng.standard_normal((B, N, D)).astype(np.float32), dtype), dtype)
+    ids = rng.integers(0, K, (B, N)).astype(np.int32)
+    ids[:, N // 3:2 * N // 3] = K // 2
+    ids[:, ::17] = -1
+    ids[:, 1::23] = K + 3
+    it = _t(ids)
+    for KO in (K, K + 2):
+        s_ids, perm = label_sort(it, K)
+        want_s = torch.zeros((B, KO, D), device="cuda")
+        want_c = torch.zeros((B, KO), dtype=torch.int32, device="cuda")
+        _C.centroid_update_sorted_indexed(x, perm, s_ids, want_s, want_c)
+        got_s = torch.full((B, KO, D), 3.5, device="cuda")
+        got_c = torch.full((B, KO), 9, dtype=torch.int32, device="cuda")
+        for _ in range(2):
+            centroid_update_sorted(x, it, K, sums_out=got_s, counts_out=got_c)
+            assert torch.equal(got_c, want_c) and torch.equal(got_s, want_s)
+    s, c = centroid_update_sorted(x[:, :0].contiguous(), it[:, :0].contiguous(), K)
+    assert not s.any() and not c.any() and s.shape == (B, K, D)

@@ -1304,8 +1304,7 @@ bool assign_uses_mfma(int dtype, int64_t D) {
 // and 1 / 2 above D = 256, where one tile also runs one workgroup per CU:
 //   (16384, 2000, 512) 77 / 109          (24000, 2000, 512) 150 / 111
 //   (131072, 2048, 512) 602 / 289        (262144, 2048, 320) 783 / 379.
-static int64_t fill_wgs(int pt, int ds2, bool exact) {
-  const int64_t cus = device_shape().cus;
+static int64_t fill_wgs(int pt, int ds2, bool exact, int64_t cus) {
   if (ds2 >= 9 && pt == 2) return cus / 2 + 1;
   if (ds2 >= 5 && pt >= 2) return cus + cus / 2;
   return (!exact && pt == 4 && ds2 == 4) ? cus : 4 * cus;
@@ -1332,7 +1331,7 @@ static bool pt8_ok(int ds2, bool pad, bool exact) {
 // at K = 4096 one or one and a half rounds lose, +8% to +12%).
 // FKC_NTILES overrides where the variant exists.
 static int choose_pt(int ds2, bool pad, bool exact, int64_t B, int64_t N,
-                     int64_t K) {
+                     int64_t K, int64_t cus) {
   const int o = ntiles_override();
   if (o == 8 && pt8_ok(ds2, pad, exact)) return o;
   if (o != 0 && o != 8 && (o * ds2 * 4 <= 64 || wide_pt(ds2, o))) return o;
@@ -1340,8 +1339,8 @@ static int choose_pt(int ds2, bool pad, bool exact, int64_t B, int64_t N,
     if (pt == 8 ? !pt8_ok(ds2, pad, exact)
                 : pt * ds2 * 4 > 64 && !wide_pt(ds2, pt))
       continue;
-    if (grid_wgs(pt, B, N) >= fill_wgs(pt, ds2, exact)) return pt;
-    if (pt == 8 && K >= 8192 && grid_wgs(8, B, N) >= 2 * device_shape().cus)
+    if (grid_wgs(pt, B, N) >= fill_wgs(pt, ds2, exact, cus)) return pt;
+    if (pt == 8 && K >= 8192 && grid_wgs(8, B, N) >= 2 * cus)
       return 8;
   }
   return 1;
@@ -1380,12 +1379,11 @@ static double round_fill(int64_t wgs, int64_t slots) {
   return (double)wgs / (double)(rounds * slots);
 }
 
-static bool use_save(const Plan& p, int64_t wgs) {
+static bool use_save(const Plan& p, int64_t wgs, int64_t cus) {
   if (p.pt != 4 || (p.ds2 != 4 && p.ds2 != 2) || p.pad || p.exact) return false;
   const int o = save_override();
   if (o >= 0) return o == 1;
   if (p.ds2 == 2) return p.kspan <= 1024;
-  const int64_t cus = device_shape().cus;
   if (p.kspan <= 2048) return true;
   if (p.kspan >= 8192) return wgs <= 2 * cus;
   return round_fill(wgs, 2 * cus) >= round_fill(wgs, 3 * cus) + 0.15;
@@ -1400,10 +1398,10 @@ static int resident_pt(int ds2) { return ds2 == 1 ? 8 : 4; }
 // workgroups than CUs leave the table fill and the first point loads
 // unhidden, and at small K the staged kernel's exact fold is as fast).
 // FKC_RESIDENT=0/1 forces it off / on where the table fits.
-static bool use_resident(const Plan& p, int64_t B, int64_t N, int64_t K) {
+static bool use_resident(const Plan& p, int64_t B, int64_t N, int64_t K,
+                         const DeviceShape& dev) {
   if (p.pad || (p.ds2 != 1 && p.ds2 != 2)) return false;
   const int64_t Kp = (K + 31) & ~int64_t{31};
-  const DeviceShape dev = device_shape();
   if (Kp > 65536 || resident_bytes(p.ds2, (int)Kp) > dev.lds_per_wg)
     return false;
   const int o = resident_override();
@@ -1423,11 +1421,12 @@ static bool use_resident(const Plan& p, int64_t B, int64_t N, int64_t K) {
 // 524288 43.3 / 39.0; K = 128: 200000 15.3 / 15.5; K = 64: 262144 15.1 / 17.2.
 // D = 64, K = 512: 200000 22.2 / 20.6, 1000000 73.3 / 62.3; K = 384: 262144
 // 18.5 / 18.4; K = 256: 262144 14.7 / 15.7.
-static bool keep_small(const Plan& p, int64_t B, int64_t N, int64_t K) {
+static bool keep_small(const Plan& p, int64_t B, int64_t N, int64_t K,
+                       int64_t cus) {
   if (p.pad || K > FKC_EXACT_MAX_K || K <= (p.ds2 == 4 ? 128 : 256) ||
       (p.ds2 != 4 && p.ds2 != 2))
     return false;
-  const int64_t cus = device_shape().cus, wgs = grid_wgs(4, B, N);
+  const int64_t wgs = grid_wgs(4, B, N);
   if (p.ds2 == 4 ? 4 * wgs < 3 * cus : wgs < 3 * cus) return false;
   const int nt = ntiles_override();
   return (nt == 0 || nt == 4) && save_override() != 0 && resident_override() != 1;
@@ -1445,7 +1444,8 @@ static bool keep_small(const Plan& p, int64_t B, int64_t N, int64_t K) {
 // eight slices 0.150 ms against 0.531 ms.  At D = 97..128 the slices fill
 // one round of resident workgroups (below).  FKC_KSPLIT forces S.
 static Plan plan_filled(int64_t B, int64_t N, int64_t K, int64_t D,
-                        bool can_slice) {
+                        bool can_slice, const DeviceShape& dev) {
+  const int64_t cus = dev.cus;
   Plan p;
   p.ds2 = (int)((D + 31) / 32);
   p.pad = D != 32 * p.ds2;
@@ -1459,23 +1459,23 @@ static Plan plan_filled(int64_t B, int64_t N, int64_t K, int64_t D,
   // (1, 262144, 768, 32) 0.0288 -> 0.0238, (4, 100000, 1000, 48) 0.0752 ->
   // 0.0695).
   p.exact = K <= FKC_EXACT_MAX_K || (p.ds2 <= 2 && K <= FKC_EXACT_MAX_K_NARROW);
-  p.pt = choose_pt(p.ds2, p.pad, p.exact, B, N, K);
+  p.pt = choose_pt(p.ds2, p.pad, p.exact, B, N, K, cus);
   p.S = 1;
   p.kspan = (int)K;
-  if (keep_small(p, B, N, K)) {
+  if (keep_small(p, B, N, K, cus)) {
     p.exact = false;
     p.save = true;
     p.pt = 4;
     return p;
   }
-  if (use_resident(p, B, N, K)) {
+  if (use_resident(p, B, N, K, dev)) {
     p.resident = true;
     p.exact = false;
     p.save = false;
     p.pt = resident_pt(p.ds2);
     return p;
   }
-  p.save = use_save(p, grid_wgs(p.pt, B, N));
+  p.save = use_save(p, grid_wgs(p.pt, B, N), cus);
   // One whole-table stage (64 KB at D = 128) where the table fits it and
   // the grid is one round of two workgroups per CU (the stage's LDS allows
   // two): one load round trip and one barrier instead of one per 64-row
@@ -1483,7 +1483,7 @@ static Plan plan_filled(int64_t B, int64_t N, int64_t K, int64_t D,
   p.whole = FKC_WHOLE_STAGE && FKC_USE_DMA && p.exact && !p.pad &&
             (p.ds2 == 1 || p.ds2 == 2 || p.ds2 == 4 || p.ds2 == 8) &&
             !wide_pt(p.ds2, p.pt) && K <= (p.ds2 <= 4 ? 256 : 128) &&
-            grid_wgs(p.pt, B, N) <= 2 * device_shape().cus;
+            grid_wgs(p.pt, B, N) <= 2 * cus;
   if (!can_slice || p.exact) return p;
   // Four tiles, not eight: on sliced-size grids four tiles on ~256
   // workgroups beat eight on 512 (N = 8192, K = 65536: 0.150 vs 0.166 ms;
@@ -1506,7 +1506,6 @@ static Plan plan_filled(int64_t B, int64_t N, int64_t K, int64_t D,
     // N = 16384, K = 32768 0.113 vs 0.122; at 8192-row slices it lost,
     // 0.215 vs 0.209, and at N = 49152 (a three-quarter round) 0.096 vs
     // 0.088).
-    const int64_t cus = device_shape().cus;
     const int64_t s3 = std::min<int64_t>(3 * cus / tiles, K / FKC_SLICE_MIN_ROWS);
     const int64_t s2 = std::min<int64_t>(2 * cus / tiles, K / FKC_SLICE_MIN_ROWS);
     S = s3;
@@ -1522,7 +1521,6 @@ static Plan plan_filled(int64_t B, int64_t N, int64_t K, int64_t D,
     // (Above D = 256 one tile per wave runs one workgroup per CU; two tiles
     // run two, and beat it wherever their grid passes fill_wgs: (16384,
     // 8192, 320) fp16 220 -> 102 us, but (1799, 16610, 408) 75 -> 106.)
-    const int64_t cus = device_shape().cus;
     for (;;) {
       const int64_t want = (wide_pt(p.ds2, pt) ? 2 : 4) * cus;
       tiles = grid_wgs(pt, B, N);
@@ -1530,7 +1528,7 @@ static Plan plan_filled(int64_t B, int64_t N, int64_t K, int64_t D,
       S = 1;
       while (tiles * S < want && K / (2 * S) >= FKC_SLICE_MIN_ROWS) S *= 2;
       if (ntiles_override() != 0 || !wide_pt(p.ds2, pt) ||
-          tiles * S >= fill_wgs(pt, p.ds2, p.exact))
+          tiles * S >= fill_wgs(pt, p.ds2, p.exact, cus))
         break;
       pt = 1;
     }
@@ -1538,7 +1536,7 @@ static Plan plan_filled(int64_t B, int64_t N, int64_t K, int64_t D,
     // Slices that still leave the chip short only pay off when the unsliced
     // grid is short too.
     if (tiles * S < want &&
-        grid_wgs(p.pt, B, N) >= fill_wgs(p.pt, p.ds2, p.exact))
+        grid_wgs(p.pt, B, N) >= fill_wgs(p.pt, p.ds2, p.exact, cus))
       return p;
   }
   const int64_t span = ((K + S - 1) / S + 127) / 128 * 128;
@@ -1547,7 +1545,7 @@ static Plan plan_filled(int64_t B, int64_t N, int64_t K, int64_t D,
   p.pt = pt;
   p.S = (int)S;
   p.kspan = (int)span;
-  p.save = use_save(p, tiles * S);
+  p.save = use_save(p, tiles * S, cus);
   return p;
 }
 
@@ -1582,11 +1580,12 @@ static double grid_model(const Plan& p, int64_t wgs, int64_t cus) {
 // 256) 50 / 34; labels are the same for every slicing.
 static Plan plan_assign(int64_t B, int64_t N, int64_t K, int64_t D,
                         bool can_slice) {
-  const Plan p = plan_filled(B, N, K, D, can_slice);
+  const DeviceShape dev = device_shape();
+  const Plan p = plan_filled(B, N, K, D, can_slice, dev);
   if (!can_slice || p.exact || p.resident || K <= FKC_EXACT_MAX_K ||
       B * N < kShortSliceMinPoints)
     return p;
-  const int64_t cus = device_shape().cus;
+  const int64_t cus = dev.cus;
   const int64_t old_wgs = grid_wgs(p.pt, B, N) * p.S;
   const double old = grid_model(p, old_wgs, cus);
   if (old_wgs >= 2 * cus || old < 17.0 || ksplit_override() != 0 ||
@@ -1607,7 +1606,7 @@ static Plan plan_assign(int64_t B, int64_t N, int64_t K, int64_t D,
       q.pt = pt;
       q.S = (int)S;
       q.kspan = (int)span;
-      q.save = use_save(q, tiles * S);
+      q.save = use_save(q, tiles * S, cus);
       const double t = grid_model(q, tiles * S, cus);
       if (t < least) {
         least = t;
@@ -1636,7 +1635,7 @@ static size_t slice_bytes(const Plan& p, int64_t B, int64_t N, Slices* sl,
 size_t assign_workspace_bytes(int64_t B, int64_t N, int64_t K, int64_t D,
                               int dtype, bool least) {
   if (!assign_uses_mfma(dtype, D) || B * N == 0 || K < 1) return 0;
-  return slice_bytes(least ? plan_filled(B, N, K, D, true)
+  return slice_bytes(least ? plan_filled(B, N, K, D, true, device_shape())
                            : plan_assign(B, N, K, D, true),
                      B, N, nullptr, nullptr);
 }

@@ -295,6 +295,10 @@ int fkc_euclid_assign(const void* x, const void* centroids, const float* x_sq,
                        nullptr, reinterpret_cast<hipStream_t>(stream));
 }
 
+int fkc_assign_reads_x_sq(int64_t D, int dtype) {
+  return assign_uses_mfma(dtype, D) ? 0 : 1;
+}
+
 size_t fkc_euclid_assign_workspace_bytes(int64_t B, int64_t N, int64_t K,
                                          int64_t D, int dtype) {
   if (shape_ok(B, N, K, D, "euclid_assign_workspace_bytes") ||

@@ -81,28 +81,30 @@ def empty_clusters(ids: torch.Tensor, K: int) -> int:
     return int(empty.item())
 
 
+def _sample_idx(x: torch.Tensor, sample_points: int, seed: int) -> torch.Tensor:
+    """int32 indices of the sample: torch.randperm(N, generator=
+    Generator(device).manual_seed(seed)) as in the reference."""
+    N = x.shape[1]
+    g = torch.Generator(device=x.device).manual_seed(int(seed))
+    idx = torch.randperm(N, generator=g, device=x.device)
+    return idx[:min(int(sample_points), N)].to(torch.int32)
+
+
 def sample_exact_inertia(x: torch.Tensor, cents: torch.Tensor, sample_points: int,
                          seed: int, chunk_n: int = 512) -> float:
     """Nearest-centroid inertia of `sample_points` points drawn without
     replacement (the same indices in every batch row), summed over rows;
-    nan when sample_points <= 0.  The indices come from
-    torch.randperm(N, generator=Generator(device).manual_seed(seed)) as in
-    the reference; the distances from fkc_sampled_inertia."""
+    nan when sample_points <= 0.  The indices come from _sample_idx, the
+    distances from fkc_sampled_inertia."""
     del chunk_n
     x, cents = _check_pair(x, cents, "sample_exact_inertia")
-    B, N, D = x.shape
-    K = cents.shape[1]
     if sample_points <= 0:
         return float("nan")
-    S = min(int(sample_points), N)
-    g = torch.Generator(device=x.device).manual_seed(int(seed))
-    idx = torch.randperm(N, generator=g, device=x.device)[:S].to(torch.int32)
-    return sampled_inertia(x, cents, idx)
+    return sampled_inertia(x, cents, _sample_idx(x, sample_points, seed))
 
 
-def sampled_inertia(x: torch.Tensor, cents: torch.Tensor, idx: torch.Tensor) -> float:
-    """Nearest-centroid inertia of the points x[:, idx] (idx int32 on x's
-    device, shared by every batch row), summed over rows (fp64)."""
+def _sampled(x: torch.Tensor, cents: torch.Tensor, idx: torch.Tensor) -> torch.Tensor:
+    """Inertia per batch row of the points x[:, idx], on the device."""
     x, cents = _check_pair(x, cents, "sampled_inertia")
     B, N, D = x.shape
     K = cents.shape[1]
@@ -118,12 +120,21 @@ def sampled_inertia(x: torch.Tensor, cents: torch.Tensor, idx: torch.Tensor) -> 
         x.data_ptr(), cents.data_ptr(), idx.data_ptr(), S, B, N, K, D, dt,
         out.data_ptr(), ws.data_ptr(), ws.numel(), _lib.stream_of(x)),
         "sampled_inertia")
-    return float(out.sum().item())
+    return out
+
+
+def sampled_inertia(x: torch.Tensor, cents: torch.Tensor, idx: torch.Tensor) -> float:
+    """Nearest-centroid inertia of the points x[:, idx] (idx int32 on x's
+    device, shared by every batch row), summed over rows (fp64)."""
+    return float(_sampled(x, cents, idx).sum().item())
 
 
 def assign_with_fixed_evaluator(x: torch.Tensor, cents: torch.Tensor) -> torch.Tensor:
-    """Labels of x against final centroids, with explicit x_sq and c_sq."""
-    return euclid_assign(x, cents.contiguous(), row_sqnorm(x), c_sq=row_sqnorm(cents))
+    """Labels of x against final centroids, with explicit x_sq (where the
+    assignment reads it: a whole pass over x) and c_sq."""
+    reads = _lib.lib.fkc_assign_reads_x_sq(x.shape[-1], _lib.dtype_code(x.dtype))
+    x_sq = row_sqnorm(x) if reads else torch.empty(0, dtype=torch.float32, device=x.device)
+    return euclid_assign(x, cents.contiguous(), x_sq, c_sq=row_sqnorm(cents))
 
 
 def evaluate(x: torch.Tensor, cents: torch.Tensor, *, sample_points: int = 4096,
@@ -133,7 +144,14 @@ def evaluate(x: torch.Tensor, cents: torch.Tensor, *, sample_points: int = 4096,
     run; its sample seed is args.seed + 1000)."""
     ids = assign_with_fixed_evaluator(x, cents)
     inertia, empty = _run(x, ids, cents, cents.shape[1], True)
-    return {"ids": ids, "inertia": float(inertia.sum().item()),
-            "inertia_per_batch": inertia.cpu().tolist(),
-            "empty_clusters": int(empty.item()),
-            "sample_exact_inertia": sample_exact_inertia(x, cents, sample_points, seed)}
+    # Everything is enqueued before anything is read: drawing the sample
+    # takes the host about twenty launches, which the GPU's work above hides.
+    # One copy brings every number back (int32 counts are exact in fp64).
+    parts = [inertia.sum().view(1), empty.to(torch.float64), inertia]
+    if sample_points > 0:
+        xd, cd = _check_pair(x, cents, "sample_exact_inertia")
+        parts.append(_sampled(xd, cd, _sample_idx(xd, sample_points, seed)).sum().view(1))
+    total, n_empty, *rest = torch.cat(parts).tolist()
+    sampled = rest.pop() if sample_points > 0 else float("nan")
+    return {"ids": ids, "inertia": total, "inertia_per_batch": rest,
+            "empty_clusters": int(n_empty), "sample_exact_inertia": sampled}

@@ -79,6 +79,12 @@ FKC_CAPI int fkc_euclid_assign(const void* x, const void* centroids,
                                fkc_stream_t stream);
 
 /*
+ * 1 where fkc_euclid_assign* reads x_sq for rows of D columns of this dtype
+ * (the fp32 route), 0 where callers may leave it out at no cost.
+ */
+FKC_CAPI int fkc_assign_reads_x_sq(int64_t D, int dtype);
+
+/*
  * Workspace variant of fkc_euclid_assign, same labels.  When the point
  * tiles of a shape cannot fill the GPU (fewer than ~1024 workgroups: N of
  * a few 100K or less with K > 512 at D = 128), the MFMA route cuts K into

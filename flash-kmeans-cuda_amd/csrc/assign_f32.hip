@@ -162,13 +162,29 @@ struct WaveWork {
 };
 
 // c_sq of the centroids whose scores a lane holds of the block at k0 (row
-// K - 1 again past K).
-template <int M>
+// K - 1 again past K).  Row by row, clamped, this costs four vector
+// instructions a value, a quarter of the vector work of a 32 x 32 block at
+// D = 37; QUADS loads four consecutive rows at a time and clamps only in the
+// last, partial block.  That branch costs the four-tile 16 x 16 loop more
+// than it saves ((1, 131072, 1024, 128) fp32 +1%), so it stays with the others
+// ((8, 34594, 1712, 19) bf16 334 -> 257 us, (1, 3000, 4000, 96) fp32 63 -> 49).
+template <int M, bool QUADS>
 __device__ inline void load_csq(const float* qb, int k0, int q, int K,
                                 float (&cq)[Shape<M>::R]) {
+  if (QUADS && k0 + M <= K) {
+    const float* p = qb + k0 + 4 * q;
 #pragma unroll
-  for (int r = 0; r < Shape<M>::R; ++r)
-    cq[r] = qb[min(k0 + Shape<M>::row(r) + 4 * q, K - 1)];
+    for (int r = 0; r < Shape<M>::R; r += 4) {
+      const Quad<FKC_F32>::Raw v =
+          *reinterpret_cast<const Quad<FKC_F32>::Raw*>(p + Shape<M>::row(r));
+#pragma unroll
+      for (int j = 0; j < 4; ++j) cq[r + j] = v[j];
+    }
+  } else {
+#pragma unroll
+    for (int r = 0; r < Shape<M>::R; ++r)
+      cq[r] = qb[min(k0 + Shape<M>::row(r) + 4 * q, K - 1)];
+  }
 }
 
 // The scores a lane holds of one block (one point, centroid rows rising with
@@ -338,7 +354,7 @@ assign_f32_kernel(const typename Elem<DT>::T* __restrict__ x,
 
   for (int t = w.kpart; t < nt; t += ks) {
     float cq[S::R];
-    load_csq<M>(qb, M * t, q, K, cq);
+    load_csq<M, M == 32 || PT == 1>(qb, M * t, q, K, cq);
     typename S::Acc acc[PT];
 #pragma unroll
     for (int p = 0; p < PT; ++p)
@@ -448,7 +464,7 @@ assign_f32_wide_kernel(const typename Elem<DT>::T* __restrict__ x,
 #pragma unroll
     for (int j = 0; j < CT; ++j) {
       float cq[S::R];
-      load_csq<M>(qb, k0 + M * j, q, K, cq);
+      load_csq<M, false>(qb, k0 + M * j, q, K, cq);
       fold_tile<M, PT>(acc[j], xs, cq, k0 + M * j, q, K, best, bidx);
     }
   }

@@ -1645,7 +1645,9 @@ int launch_assign_mfma(const void* x, const void* c, const float* c_sq,
                        int64_t D, int dtype, const int32_t* ctrl,
                        hipStream_t s, hipEvent_t ev0, hipEvent_t ev1,
                        void* ws, size_t ws_bytes) {
-  const Plan p = plan_assign(B, N, K, D, ws != nullptr);
+  Plan p = plan_assign(B, N, K, D, ws != nullptr);
+  if (slice_bytes(p, B, N, nullptr, nullptr) > ws_bytes)
+    p = plan_filled(B, N, K, D, ws != nullptr, device_shape());
   if (p.resident) {
     using RL = int (*)(const void*, const void*, const float*, int32_t*,
                        int64_t, int64_t, int64_t, const int32_t*, hipStream_t,

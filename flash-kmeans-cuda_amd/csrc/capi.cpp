@@ -226,11 +226,11 @@ struct LoopBuffers {
   size_t asg_ws_bytes = 0;
 };
 
-// slices: with room for a sliced assign's partial winners (their plan is
-// the assign's own; without them it runs unsliced, with the same labels).
+// least: with the assign's least workspace (launch_assign takes the plan that
+// fits what it is given; labels are the same for every slicing).
 LoopBuffers carve_loop(void* ws, int64_t B, int64_t N, int64_t K, int64_t D,
                        int dtype, int max_iters, size_t* total,
-                       bool slices = true) {
+                       bool least = false) {
   Carve c(ws);
   LoopBuffers L;
   if (!assign_uses_mfma(dtype, D)) L.x_sq = c.take<float>((size_t)B * N);
@@ -245,7 +245,7 @@ LoopBuffers carve_loop(void* ws, int64_t B, int64_t N, int64_t K, int64_t D,
   L.sort_ws = c.take<char>(L.sort_ws_bytes);
   L.upd_ws_bytes = update_workspace_bytes(B, N, D);
   L.upd_ws = c.take<char>(L.upd_ws_bytes);
-  L.asg_ws_bytes = slices ? assign_workspace_bytes(B, N, K, D, dtype) : 0;
+  L.asg_ws_bytes = assign_workspace_bytes(B, N, K, D, dtype, least);
   L.asg_ws = L.asg_ws_bytes ? c.take<char>(L.asg_ws_bytes) : nullptr;
   if (total) *total = c.used;
   return L;
@@ -319,7 +319,12 @@ int fkc_euclid_assign_ws(const void* x, const void* centroids,
   if (!x || !centroids || !c_sq || !cluster_ids)
     return fail(FKC_ERR_INVALID, "euclid_assign_ws: null pointer argument");
   const size_t need = assign_workspace_bytes(B, N, K, D, dtype);
-  if (need == 0)
+  const bool fits = workspace && workspace_bytes >= need &&
+                    reinterpret_cast<uintptr_t>(workspace) % kWorkspaceAlign == 0;
+  // Slices that only shorten an underfilled launch are not asked for: such a
+  // shape also runs, unsliced, with no workspace.
+  if (need == 0 ||
+      (!fits && assign_workspace_bytes(B, N, K, D, dtype, true) == 0))
     return launch_assign(x, centroids, x_sq, c_sq, cluster_ids, B, N, K, D,
                          dtype, nullptr, reinterpret_cast<hipStream_t>(stream));
   if (!workspace || workspace_bytes < need)
@@ -556,9 +561,8 @@ size_t lloyd_least_workspace_bytes(int64_t B, int64_t N, int64_t K, int64_t D,
                                    int dtype, int max_iters) {
   if (B <= 0 || N <= 0 || K < 1 || D < 1) return 256;
   size_t total = 0;
-  carve_loop(nullptr, B, N, K, D, dtype, max_iters, &total, false);
-  return total +
-         align_up(assign_workspace_bytes(B, N, K, D, dtype, true), 256);
+  carve_loop(nullptr, B, N, K, D, dtype, max_iters, &total, true);
+  return total;
 }
 
 // fkc_kmeans_lloyd (init == centroids), fkc_kmeans_lloyd_from and the
@@ -567,8 +571,7 @@ int lloyd_run(const void* x, const void* init, void* centroids,
               int32_t* cluster_ids, int64_t B, int64_t N, int64_t K,
               int64_t D, int dtype, int max_iters, float tol, void* workspace,
               size_t workspace_bytes, fkc_stream_t stream,
-              int32_t* n_iters_dev, int32_t* n_iters_host, bool profile,
-              bool fixed_ws) {
+              int32_t* n_iters_dev, int32_t* n_iters_host, bool profile) {
   g_err[0] = 0;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   if (int rc = shape_ok(B, N, K, D, "kmeans_lloyd")) return rc;
@@ -594,10 +597,10 @@ int lloyd_run(const void* x, const void* init, void* centroids,
     return fail(FKC_ERR_INVALID, "kmeans_lloyd: null pointer argument");
   size_t need = 0;
   carve_loop(nullptr, B, N, K, D, dtype, max_iters, &need);
-  // A workspace of fixed size (the static one) gives up the assign's slices
-  // before it refuses a shape.
-  const bool slices = !fixed_ws || need <= workspace_bytes;
-  if (!slices) carve_loop(nullptr, B, N, K, D, dtype, max_iters, &need, false);
+  // A workspace of fixed size (the static one, or one that a caller sized for
+  // its largest shape) gives up the assign's short slices before it is refused.
+  const bool least = need > workspace_bytes;
+  if (least) carve_loop(nullptr, B, N, K, D, dtype, max_iters, &need, true);
   if (!workspace || workspace_bytes < need)
     return fail(FKC_ERR_WORKSPACE, "kmeans_lloyd: workspace %zu < %zu bytes",
                 workspace_bytes, need);
@@ -605,7 +608,7 @@ int lloyd_run(const void* x, const void* init, void* centroids,
     return fail(FKC_ERR_WORKSPACE, "kmeans_lloyd: workspace not %d-byte aligned",
                 kWorkspaceAlign);
   LoopBuffers L =
-      carve_loop(workspace, B, N, K, D, dtype, max_iters, nullptr, slices);
+      carve_loop(workspace, B, N, K, D, dtype, max_iters, nullptr, least);
 
   const bool check = tol > 0.f;
   const int32_t* ctrl = check ? L.ctrl : nullptr;

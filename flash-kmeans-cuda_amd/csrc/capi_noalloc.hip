@@ -76,8 +76,7 @@ int fkc_kmeans_lloyd_noalloc(const void* x, const void* init_centroids,
   if (int rc = fkc::scratch_on_current_device(&ws)) return rc;
   return fkc::lloyd_run(x, init_centroids, centroids, cluster_ids, B, N, K, D,
                         dtype, max_iters, tol, ws, fkc::kScratchBytes, stream,
-                        n_iters_dev, n_iters_host, /*profile=*/false,
-                        /*fixed_ws=*/true);
+                        n_iters_dev, n_iters_host, /*profile=*/false);
 }
 
 }  // extern "C"

@@ -48,8 +48,9 @@ size_t assign_workspace_bytes(int64_t B, int64_t N, int64_t K, int64_t D,
                               int dtype, bool least = false);
 // ev0 / ev1 (optional, both or neither): timing events of the launch; on
 // the MFMA route the dispatch packets stamp them (no extra stream packets).
-// ws (optional, assign_workspace_bytes): with it the MFMA route may slice K;
-// without it the launch is never sliced.
+// ws (optional, assign_workspace_bytes): with it the MFMA route may slice K,
+// with the least one as far as that reaches; without it the launch is never
+// sliced.
 int launch_assign(const void* x, const void* c, const float* x_sq,
                   const float* c_sq, int32_t* ids, int64_t B, int64_t N,
                   int64_t K, int64_t D, int dtype, const int32_t* ctrl,
@@ -205,8 +206,9 @@ int launch_quality(const void* x, const void* c, const int32_t* ids,
                    hipStream_t s, const int32_t* sidx = nullptr,
                    int64_t sN = 0);
 // Nearest-centroid inertia of the S sampled points idx[0..S) of every row.
+// slices: with room for the assign's slices (sampled_inertia runs without).
 size_t sample_workspace_bytes(int64_t B, int64_t S, int64_t K, int64_t D,
-                              int dtype);
+                              int dtype, bool slices = true);
 int launch_sampled_inertia(const void* x, const void* c, const int32_t* idx,
                            int64_t S, int64_t B, int64_t N, int64_t K,
                            int64_t D, int dtype, double* inertia, void* ws,
@@ -214,14 +216,13 @@ int launch_sampled_inertia(const void* x, const void* c, const int32_t* idx,
 
 // ---------------------------------------------------------------- loop
 // The Lloyd loop behind fkc_kmeans_lloyd*; profile = false ignores the
-// profiling hook (creates no events); fixed_ws: a workspace too small for
-// the assign's slices runs it unsliced instead of being refused.
+// profiling hook (creates no events).  A workspace of at least
+// lloyd_least_workspace_bytes is enough; the assign slices as it fits.
 int lloyd_run(const void* x, const void* init, void* centroids,
               int32_t* cluster_ids, int64_t B, int64_t N, int64_t K,
               int64_t D, int dtype, int max_iters, float tol, void* workspace,
               size_t workspace_bytes, fkc_stream_t stream,
-              int32_t* n_iters_dev, int32_t* n_iters_host, bool profile,
-              bool fixed_ws = false);
+              int32_t* n_iters_dev, int32_t* n_iters_host, bool profile);
 // The loop's workspace with assign_workspace_bytes(..., least).
 size_t lloyd_least_workspace_bytes(int64_t B, int64_t N, int64_t K, int64_t D,
                                  int dtype, int max_iters);

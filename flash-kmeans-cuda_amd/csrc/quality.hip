@@ -214,14 +214,14 @@ size_t quality_workspace_bytes(int64_t B, int64_t N, int64_t K) {
 }
 
 size_t sample_workspace_bytes(int64_t B, int64_t S, int64_t K, int64_t D,
-                              int dtype) {
+                              int dtype, bool slices) {
   Carve c(nullptr);
   c.take<char>((size_t)B * S * D * dtype_size(dtype));  // sampled rows
   c.take<float>((size_t)B * S);                         // their x_sq
   c.take<float>((size_t)B * K);                         // c_sq
   c.take<int32_t>((size_t)B * S);                       // their labels
-  c.take<char>(assign_workspace_bytes(B, S, K, D, dtype));
   c.take<char>(quality_workspace_bytes(B, S, K));
+  if (slices) c.take<char>(assign_workspace_bytes(B, S, K, D, dtype));
   return c.used;
 }
 
@@ -229,7 +229,9 @@ int launch_sampled_inertia(const void* x, const void* c, const int32_t* idx,
                            int64_t S, int64_t B, int64_t N, int64_t K,
                            int64_t D, int dtype, double* inertia, void* ws,
                            size_t ws_bytes, hipStream_t s) {
-  const size_t need = sample_workspace_bytes(B, S, K, D, dtype);
+  // Without room for the assign's slices it runs unsliced.
+  const bool slices = ws_bytes >= sample_workspace_bytes(B, S, K, D, dtype);
+  const size_t need = sample_workspace_bytes(B, S, K, D, dtype, false);
   if (ws == nullptr || ws_bytes < need)
     return fail(FKC_ERR_WORKSPACE, "sampled_inertia: workspace %zu < %zu bytes",
                 ws_bytes, need);
@@ -242,10 +244,11 @@ int launch_sampled_inertia(const void* x, const void* c, const int32_t* idx,
   float* xs_sq = cv.take<float>((size_t)B * S);
   float* c_sq = cv.take<float>((size_t)B * K);
   int32_t* lab = cv.take<int32_t>((size_t)B * S);
-  const size_t abytes = assign_workspace_bytes(B, S, K, D, dtype);
-  void* aws = abytes ? cv.take<char>(abytes) : nullptr;
   const size_t qbytes = quality_workspace_bytes(B, S, K);
   void* qws = cv.take<char>(qbytes);
+  const size_t abytes =
+      slices ? assign_workspace_bytes(B, S, K, D, dtype) : 0;
+  void* aws = abytes ? cv.take<char>(abytes) : nullptr;
   const int row_bytes = (int)(D * dtype_size(dtype));
   hipLaunchKernelGGL(sample_gather_kernel,
                      dim3((unsigned)((S + 3) / 4), (unsigned)B), dim3(256), 0,

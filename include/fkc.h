@@ -93,7 +93,10 @@ FKC_CAPI int fkc_assign_reads_x_sq(int64_t D, int dtype);
  * workspace holds the partial winners, 8 bytes per point and slice.
  * fkc_euclid_assign_workspace_bytes returns the bytes needed (0: the shape
  * is not sliced and the workspace may be NULL); the workspace is 256-byte
- * aligned and may be reused once the call's stream work is done.  Same
+ * aligned and may be reused once the call's stream work is done.  Shapes
+ * whose slices would be shorter than 2048 rows also run, unsliced and
+ * slower, with a workspace that does not hold them (fkc_kmeans_lloyd and
+ * fkc_sampled_inertia likewise).  Same
  * reference interfaces as fkc_euclid_assign (flash_kmeans_cuda.h:41-46,
  * bindings.cpp:43-63); the slicing has no counterpart there (the reference
  * picks among tile shapes per dtype, D and K, assign_sm80.cu:707-1111).

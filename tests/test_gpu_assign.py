@@ -351,6 +351,51 @@ def test_sliced_assign_workspace_errors(monkeypatch):
     assert _lib.lib.fkc_euclid_assign_workspace_bytes(1, 5000, 300, 128, 1) == 0
 
 
+@pytest.mark.parametrize("B,N,K,D", [(1, 1000, 4000, 128), (2, 1501, 2100, 200)])
+def test_short_slices_are_not_demanded(monkeypatch, B, N, K, D):
+    """A workspace that holds a shape's sums and sort, but not the slices that
+    only shorten an underfilled launch, is accepted by every entry point, with
+    the same labels; one below that is refused."""
+    from flash_kmeans_cuda import _lib
+    L = _lib.lib
+    for v in ("FKC_KSPLIT", "FKC_NTILES"):
+        monkeypatch.delenv(v, raising=False)
+    g = torch.Generator(device="cuda").manual_seed(K)
+    x = torch.randn(B, N, D, device="cuda", generator=g).half()
+    c = x[:, torch.randint(0, N, (K,), device="cuda", generator=g)].contiguous()
+    csq = c.float().pow(2).sum(-1)
+    st = _lib.stream_of(x)
+    need = L.fkc_euclid_assign_workspace_bytes(B, N, K, D, 1)
+    assert need > 0
+    ws = torch.empty(need + 256, dtype=torch.uint8, device="cuda")
+    got = []
+    for p, n in ((ws.data_ptr(), need), (ws.data_ptr(), need - 1), (None, 0),
+                 (ws.data_ptr() + 8, need)):
+        ids = torch.empty((B, N), dtype=torch.int32, device="cuda")
+        assert L.fkc_euclid_assign_ws(x.data_ptr(), c.data_ptr(), None, csq.data_ptr(),
+                                      ids.data_ptr(), B, N, K, D, 1, p, n, st) == 0
+        got.append(ids)
+    assert all(torch.equal(got[0], o) for o in got[1:])
+
+    def lloyd(n):
+        cent, ids = c.clone(), torch.empty((B, N), dtype=torch.int32, device="cuda")
+        w = torch.empty(n, dtype=torch.uint8, device="cuda")
+        it = torch.empty(1, dtype=torch.int32, device="cuda")
+        rc = L.fkc_kmeans_lloyd(x.data_ptr(), cent.data_ptr(), ids.data_ptr(), B, N, K, D, 1, 2,
+                                0.0, w.data_ptr(), n, st, it.data_ptr(), None)
+        return rc, cent, ids
+
+    full = L.fkc_kmeans_workspace_bytes(B, N, K, D, 1, 2)
+    monkeypatch.setenv("FKC_KSPLIT", "1")
+    least = L.fkc_kmeans_workspace_bytes(B, N, K, D, 1, 2)
+    monkeypatch.delenv("FKC_KSPLIT")
+    assert least < full
+    a, b = lloyd(full), lloyd(least)
+    assert a[0] == 0 and b[0] == 0
+    assert torch.equal(a[1], b[1]) and torch.equal(a[2], b[2])
+    assert lloyd(least - 256)[0] == 2
+
+
 @pytest.mark.parametrize("B,N,K,D,dtype", [(1, 140000, 40, 24, "f32"), (1, 140000, 33, 37, "f16")])
 def test_vector_route_one_lane_per_point(B, N, K, D, dtype):
     """The VALU route with one lane per point (grids of >= 512 workgroups:

@@ -351,6 +351,26 @@ def test_sliced_assign_workspace_errors(monkeypatch):
     assert _lib.lib.fkc_euclid_assign_workspace_bytes(1, 5000, 300, 128, 1) == 0
 
 
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("D", [1, 37, 64, 66, 128, 513])
+def test_row_norms_do_not_depend_on_the_rows_per_wave(dtype, D):
+    """Many rows (four per wave, a ragged last group, also off the vector
+    alignment) against the same rows in small calls (one per wave), bit for
+    bit, and a float64 sum."""
+    from flash_kmeans_cuda.ops import row_sqnorm
+    dt = {"f32": torch.float32, "f16": torch.float16, "bf16": torch.bfloat16}[dtype]
+    g = torch.Generator(device="cuda").manual_seed(D)
+    rows = 32768 + 3
+    flat = torch.randn(rows * D + 1, device="cuda", generator=g).to(dt)
+    for x in (flat[:-1].view(1, rows, D), flat[1:].view(1, rows, D)):
+        got = row_sqnorm(x)
+        parts = torch.cat([row_sqnorm(p) for p in x.split(16384, dim=1)], dim=1)
+        assert torch.equal(got, parts)
+        want = x.double().pow(2).sum(-1)
+        # at most D / 64 + 2 roundings in a lane and 6 in the tree, 2^-24 each
+        assert ((got.double() - want).abs() <= (D / 64 + 8) * 2.0 ** -24 * want).all()
+
+
 @pytest.mark.parametrize("B,N,K,D", [(1, 1000, 4000, 128), (2, 1501, 2100, 200)])
 def test_short_slices_are_not_demanded(monkeypatch, B, N, K, D):
     """A workspace that holds a shape's sums and sort, but not the slices that

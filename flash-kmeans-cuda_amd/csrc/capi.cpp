@@ -8,6 +8,7 @@
 // throwing TORCH_CHECK errors across the ABI.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
@@ -299,12 +300,30 @@ int fkc_assign_reads_x_sq(int64_t D, int dtype) {
   return assign_uses_mfma(dtype, D) ? 0 : 1;
 }
 
-size_t fkc_euclid_assign_workspace_bytes(int64_t B, int64_t N, int64_t K,
-                                         int64_t D, int dtype) {
+size_t fkc_euclid_assign_fast_workspace_bytes(int64_t B, int64_t N, int64_t K,
+                                              int64_t D, int dtype) {
   if (shape_ok(B, N, K, D, "euclid_assign_workspace_bytes") ||
       dtype_ok(dtype, "euclid_assign_workspace_bytes"))
     return 0;
   return assign_workspace_bytes(B, N, K, D, dtype);
+}
+
+// What fkc_euclid_assign_ws asks for: the whole slices, or the short ones
+// where they do with less; 0 where only short slices are planned.  (A caller
+// with room for the whole slices is spared the second plan.)
+static size_t assign_required_bytes(int64_t B, int64_t N, int64_t K, int64_t D,
+                                    int dtype, size_t given = 0) {
+  const size_t whole = assign_workspace_bytes(B, N, K, D, dtype, true);
+  if (whole <= given) return whole;
+  return std::min(whole, assign_workspace_bytes(B, N, K, D, dtype));
+}
+
+size_t fkc_euclid_assign_workspace_bytes(int64_t B, int64_t N, int64_t K,
+                                         int64_t D, int dtype) {
+  const size_t fast = fkc_euclid_assign_fast_workspace_bytes(B, N, K, D, dtype);
+  if (fast == 0) return 0;
+  const size_t need = assign_required_bytes(B, N, K, D, dtype);
+  return need ? need : fast;
 }
 
 int fkc_euclid_assign_ws(const void* x, const void* centroids,
@@ -318,22 +337,18 @@ int fkc_euclid_assign_ws(const void* x, const void* centroids,
   if (B * N == 0) return FKC_OK;
   if (!x || !centroids || !c_sq || !cluster_ids)
     return fail(FKC_ERR_INVALID, "euclid_assign_ws: null pointer argument");
-  const size_t need = assign_workspace_bytes(B, N, K, D, dtype);
-  const bool fits = workspace && workspace_bytes >= need &&
-                    reinterpret_cast<uintptr_t>(workspace) % kWorkspaceAlign == 0;
-  // Slices that only shorten an underfilled launch are not asked for: such a
-  // shape also runs, unsliced, with no workspace.
-  if (need == 0 ||
-      (!fits && assign_workspace_bytes(B, N, K, D, dtype, true) == 0))
-    return launch_assign(x, centroids, x_sq, c_sq, cluster_ids, B, N, K, D,
-                         dtype, nullptr, reinterpret_cast<hipStream_t>(stream));
-  if (!workspace || workspace_bytes < need)
+  const size_t need =
+      assign_required_bytes(B, N, K, D, dtype, workspace_bytes);
+  const bool aligned =
+      reinterpret_cast<uintptr_t>(workspace) % kWorkspaceAlign == 0;
+  if (need && (!workspace || workspace_bytes < need))
     return fail(FKC_ERR_WORKSPACE, "euclid_assign_ws: workspace %zu < %zu bytes",
                 workspace_bytes, need);
-  if (reinterpret_cast<uintptr_t>(workspace) % kWorkspaceAlign != 0)
+  if (need && !aligned)
     return fail(FKC_ERR_WORKSPACE,
                 "euclid_assign_ws: workspace not %d-byte aligned",
                 kWorkspaceAlign);
+  if (!aligned) workspace = nullptr;  // nothing is asked for: unsliced
   return launch_assign(x, centroids, x_sq, c_sq, cluster_ids, B, N, K, D, dtype,
                        nullptr, reinterpret_cast<hipStream_t>(stream), nullptr,
                        nullptr, workspace, workspace_bytes);

@@ -62,7 +62,7 @@ def euclid_assign(x: torch.Tensor, centroids: torch.Tensor, x_sq: torch.Tensor,
         _contig(x_sq)
         xsq_ptr = x_sq.data_ptr()
     dt = _lib.dtype_code(x.dtype)
-    need = _lib.lib.fkc_euclid_assign_workspace_bytes(B, N, K, D, dt)
+    need = _lib.lib.fkc_euclid_assign_fast_workspace_bytes(B, N, K, D, dt)
     if need == 0:
         _lib.check(_lib.lib.fkc_euclid_assign(
             x.data_ptr(), centroids.data_ptr(), xsq_ptr, c_sq.data_ptr(),

@@ -33,6 +33,7 @@ SIGNATURES = {
     "fkc_euclid_assign": (_int, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _vp]),
     "fkc_assign_reads_x_sq": (_int, [_i64, _int]),
     "fkc_euclid_assign_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64, _int]),
+    "fkc_euclid_assign_fast_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64, _int]),
     "fkc_euclid_assign_ws": (_int, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _vp, _sz, _vp]),
     "fkc_row_sqnorm": (_int, [_vp, _vp, _i64, _i64, _int, _vp]),
     "fkc_label_sort_workspace_bytes": (_sz, [_i64, _i64, _i64]),

@@ -122,7 +122,7 @@ at::Tensor euclid_assign_out(const at::Tensor& x, const at::Tensor& centroids,
     TORCH_CHECK(x_sq.is_contiguous(), "all tensors must be contiguous");
     xsq = x_sq.data_ptr<float>();
   }
-  const size_t need = fkc_euclid_assign_workspace_bytes(B, N, K, D, dtype_code(x));
+  const size_t need = fkc_euclid_assign_fast_workspace_bytes(B, N, K, D, dtype_code(x));
   if (need == 0) {
     check_rc(fkc_euclid_assign(x.data_ptr(), centroids.data_ptr(), xsq, c_sq.data_ptr<float>(),
                                cluster_ids.data_ptr<int32_t>(), B, N, K, D, dtype_code(x),

@@ -93,10 +93,13 @@ FKC_CAPI int fkc_assign_reads_x_sq(int64_t D, int dtype);
  * workspace holds the partial winners, 8 bytes per point and slice.
  * fkc_euclid_assign_workspace_bytes returns the bytes needed (0: the shape
  * is not sliced and the workspace may be NULL); the workspace is 256-byte
- * aligned and may be reused once the call's stream work is done.  Shapes
- * whose slices would be shorter than 2048 rows also run, unsliced and
- * slower, with a workspace that does not hold them (fkc_kmeans_lloyd and
- * fkc_sampled_inertia likewise).  Same
+ * aligned and may be reused once the call's stream work is done.  Slices
+ * shorter than 2048 rows are taken only where they are faster, and are not
+ * demanded: with fkc_euclid_assign_fast_workspace_bytes (never less) the
+ * launch takes them; with less it takes 2048-row ones where K and the shape
+ * give any (what fkc_euclid_assign_workspace_bytes then asks for), and runs
+ * unsliced where they do not, also with a NULL workspace.  (fkc_kmeans_lloyd
+ * and fkc_sampled_inertia accept smaller workspaces likewise.)  Same
  * reference interfaces as fkc_euclid_assign (flash_kmeans_cuda.h:41-46,
  * bindings.cpp:43-63); the slicing has no counterpart there (the reference
  * picks among tile shapes per dtype, D and K, assign_sm80.cu:707-1111).
@@ -104,6 +107,9 @@ FKC_CAPI int fkc_assign_reads_x_sq(int64_t D, int dtype);
 FKC_CAPI size_t fkc_euclid_assign_workspace_bytes(int64_t B, int64_t N,
                                                   int64_t K, int64_t D,
                                                   int dtype);
+FKC_CAPI size_t fkc_euclid_assign_fast_workspace_bytes(int64_t B, int64_t N,
+                                                       int64_t K, int64_t D,
+                                                       int dtype);
 FKC_CAPI int fkc_euclid_assign_ws(const void* x, const void* centroids,
                                   const float* x_sq, const float* c_sq,
                                   int32_t* cluster_ids, int64_t B, int64_t N,

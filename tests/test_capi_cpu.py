@@ -186,6 +186,27 @@ def test_assign_slice_plan(monkeypatch):
     assert f(1, 80000, 70000, 16, 1) == 0
 
 
+# Shapes whose whole slices (at least 2048 rows) need the given bytes, 8 per
+# point and slice, and whose shorter, faster slices need more.
+WHOLE_SLICE_BYTES = [
+    (1, 1000, 4096, 128, 16384), (1, 4096, 4096, 128, 65536), (1, 8192, 8192, 128, 262144),
+    (1, 1000, 8192, 64, 32256), (1, 2000, 16384, 256, 128000),
+]
+
+
+@pytest.mark.parametrize("B,N,K,D,nbytes", WHOLE_SLICE_BYTES)
+def test_assign_asks_for_whole_slices_only(monkeypatch, B, N, K, D, nbytes):
+    from flash_kmeans_cuda import _lib
+    monkeypatch.delenv("FKC_KSPLIT", raising=False)
+    monkeypatch.delenv("FKC_NTILES", raising=False)
+    L = _lib.lib
+    assert L.fkc_euclid_assign_workspace_bytes(B, N, K, D, 1) == nbytes
+    assert L.fkc_euclid_assign_fast_workspace_bytes(B, N, K, D, 1) > nbytes
+    fake = ctypes.c_void_p(0x1000)  # refused before any pointer is used
+    assert L.fkc_euclid_assign_ws(fake, fake, None, fake, fake, B, N, K, D, 1, fake,
+                                  nbytes - 1, None) == 2
+
+
 def test_workspace_sizes():
     from flash_kmeans_cuda import _lib
     L = _lib.lib

@@ -416,6 +416,37 @@ def test_short_slices_are_not_demanded(monkeypatch, B, N, K, D):
     assert lloyd(least - 256)[0] == 2
 
 
+@pytest.mark.parametrize("B,N,K,D,nbytes", [
+    (1, 1000, 4096, 128, 16384), (1, 4096, 4096, 128, 65536), (1, 8192, 8192, 128, 262144),
+    (1, 1000, 8192, 64, 32256), (1, 2000, 16384, 256, 128000),
+])
+def test_whole_slices_are_enough(monkeypatch, B, N, K, D, nbytes):
+    """Where K gives whole slices (nbytes: 8 per point and slice), a workspace
+    that holds those, but not the shorter ones that are faster, is accepted
+    with the same labels, and nothing smaller is."""
+    from flash_kmeans_cuda import _lib
+    L = _lib.lib
+    for v in ("FKC_KSPLIT", "FKC_NTILES"):
+        monkeypatch.delenv(v, raising=False)
+    g = torch.Generator(device="cuda").manual_seed(K + D)
+    x = torch.randn(B, N, D, device="cuda", generator=g).half()
+    c = torch.randn(B, K, D, device="cuda", generator=g).half()
+    c[:, K - 1] = c[:, 7]
+    csq = c.float().pow(2).sum(-1)
+    fast = L.fkc_euclid_assign_fast_workspace_bytes(B, N, K, D, 1)
+    ws = torch.empty(fast, dtype=torch.uint8, device="cuda")
+    args = (x.data_ptr(), c.data_ptr(), None, csq.data_ptr())
+    got = []
+    for n in (nbytes, fast - 1, fast):
+        ids = torch.empty((B, N), dtype=torch.int32, device="cuda")
+        assert L.fkc_euclid_assign_ws(*args, ids.data_ptr(), B, N, K, D, 1, ws.data_ptr(), n,
+                                      _lib.stream_of(x)) == 0
+        got.append(ids)
+    assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
+    assert L.fkc_euclid_assign_ws(*args, ids.data_ptr(), B, N, K, D, 1, ws.data_ptr(),
+                                  nbytes - 1, _lib.stream_of(x)) == 2
+
+
 @pytest.mark.parametrize("B,N,K,D,dtype", [(1, 140000, 40, 24, "f32"), (1, 140000, 33, 37, "f16")])
 def test_vector_route_one_lane_per_point(B, N, K, D, dtype):
     """The VALU route with one lane per point (grids of >= 512 workgroups:

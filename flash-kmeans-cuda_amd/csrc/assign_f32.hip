@@ -38,6 +38,8 @@
 #include "device_util.hpp"
 #include "fkc_internal.hpp"
 
+#include <algorithm>
+
 #include <float.h>
 
 namespace fkc {
@@ -125,6 +127,9 @@ struct Shape<16> {
   }
   // Accumulator register r of lane group q holds centroid row(r) + 4 q.
   __device__ static constexpr int row(int r) { return r; }
+  // Register and lane of the diagonal's entry col.
+  __device__ static int diag_reg(int col) { return col & 3; }
+  __device__ static int diag_lane(int col) { return 16 * (col >> 2) + col; }
 };
 
 template <>
@@ -147,6 +152,8 @@ struct Shape<32> {
     o[3] = __uint_as_float(b[1]);
   }
   __device__ static constexpr int row(int r) { return 8 * (r / 4) + r % 4; }
+  __device__ static int diag_reg(int col) { return 4 * (col >> 3) + (col & 3); }
+  __device__ static int diag_lane(int col) { return 32 * (col >> 2 & 1) + col; }
 };
 
 // Where a wave's work lies: ks (1, 2 or 4) waves of the workgroup share one
@@ -277,25 +284,27 @@ __device__ inline void merge_store(float (&best)[PT], int (&bidx)[PT], int ks,
   if (lane < M * PT && w.n0 + lane < N) ids[w.n0 + lane] = i;
 }
 
-// ||x_n||^2 of the point tiles' points: given, or as the chain of v * v.
-template <int DT, int M, int PT>
-__device__ inline void point_norms(const typename Elem<DT>::T* xb,
-                                   const float* x_sq, int n0, int N, int D,
+// ||x_n||^2 of the points of tile p, given.
+template <int M, int PT>
+__device__ inline void given_norms(const float* x_sq, int n0, int N,
                                    float (&xs)[PT]) {
-  const int col = threadIdx.x % M;
 #pragma unroll
-  for (int p = 0; p < PT; ++p) {
-    const int n = min(n0 + M * p + col, N - 1);
-    if (x_sq != nullptr) {
-      xs[p] = x_sq[n];
-    } else {
-      xs[p] = 0.f;
-      for (int d = 0; d < D; ++d) {
-        const float v = Elem<DT>::load(xb[(size_t)n * D + d]);
-        xs[p] = fmaf(v, v, xs[p]);
-      }
-    }
-  }
+  for (int p = 0; p < PT; ++p)
+    xs[p] = x_sq[min(n0 + M * p + (int)threadIdx.x % M, N - 1)];
+}
+
+// ||x_n||^2 computed: points scored against themselves give the chain of
+// v * v on the block's diagonal; every lane takes its own point's entry.  (A
+// loop over the features in the vector unit waits for a round trip each: (1,
+// 35, 5, 768) fp32 283 us of 300.)
+template <int M>
+__device__ inline float diagonal(const typename Shape<M>::Acc& acc) {
+  using S = Shape<M>;
+  const int col = threadIdx.x % M;
+  float v = acc[0];
+#pragma unroll
+  for (int r = 1; r < S::R; ++r) v = S::diag_reg(col) == r ? acc[r] : v;
+  return __shfl(v, S::diag_lane(col), 64);
 }
 
 // D <= 512.  M: instruction shape; G: feature groups a row takes (D <= FG G),
@@ -345,7 +354,19 @@ assign_f32_kernel(const typename Elem<DT>::T* __restrict__ x,
   }
   float xs[PT], best[PT];
   int bidx[PT];
-  point_norms<DT, M, PT>(xb, x_sq ? x_sq + (size_t)b * N : nullptr, w.n0, N, D, xs);
+  if (x_sq != nullptr) {
+    given_norms<M, PT>(x_sq + (size_t)b * N, w.n0, N, xs);
+  } else {
+#pragma unroll
+    for (int p = 0; p < PT; ++p) {
+      typename S::Acc acc = {};
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) acc = S::mfma(bx[p][g][s], bx[p][g][s], acc);
+      xs[p] = diagonal<M>(acc);
+    }
+  }
 #pragma unroll
   for (int p = 0; p < PT; ++p) {
     best[p] = FLT_MAX;
@@ -379,10 +400,13 @@ assign_f32_kernel(const typename Elem<DT>::T* __restrict__ x,
 }
 
 // Any D (used above 512, where a point tile's operands no longer fit the
-// registers): both operands stream, and 4 x 4 blocks of 16 x 16 scores per
-// wave give each quad four uses.  (1, 20000, 500, 768) fp32 974 us with the
-// vector kernel, 289 with this one; fp16 2362 and 284.
-template <int DT>
+// registers): both operands stream, and CT x PT blocks of 16 x 16 scores per
+// wave give each quad CT or PT uses.  4 x 4 blocks where N and K fill them:
+// (1, 20000, 500, 768) fp32 974 us with the vector kernel, 289 with this one;
+// fp16 2362 and 284.  Smaller blocks (plan_wide) for few points or few
+// centroids, with PD groups of quads in flight: with one in flight a wave
+// waits for a round trip per group.
+template <int DT, int PT, int CT, int PD>
 __global__ void __launch_bounds__(FT, 2)
 assign_f32_wide_kernel(const typename Elem<DT>::T* __restrict__ x,
                        const typename Elem<DT>::T* __restrict__ c,
@@ -393,7 +417,7 @@ assign_f32_wide_kernel(const typename Elem<DT>::T* __restrict__ x,
   using T = typename Elem<DT>::T;
   using Raw = typename Quad<DT>::Raw;
   using S = Shape<16>;
-  constexpr int M = 16, PT = 4, CT = 4;
+  constexpr int M = 16;
   if (loop_done(ctrl)) return;
   const int lane = threadIdx.x & 63, col = lane % M, q = lane / M;
   const int b = blockIdx.y;
@@ -403,7 +427,6 @@ assign_f32_wide_kernel(const typename Elem<DT>::T* __restrict__ x,
   const float* qb = c_sq + (size_t)b * K;
   float xs[PT], best[PT];
   int bidx[PT];
-  point_norms<DT, M, PT>(xb, x_sq ? x_sq + (size_t)b * N : nullptr, w.n0, N, D, xs);
   const T* xrow[PT];
 #pragma unroll
   for (int p = 0; p < PT; ++p) {
@@ -411,7 +434,58 @@ assign_f32_wide_kernel(const typename Elem<DT>::T* __restrict__ x,
     bidx[p] = 0;
     xrow[p] = xb + (size_t)min(w.n0 + M * p + col, N - 1) * D;
   }
-  const int nfull = D / S::FG;
+  const int nfull = D / S::FG;  // > PD
+  const bool rest = D % S::FG != 0;
+
+  // The groups of a row in order: load(i, g, whole) fills slot i of PD with
+  // group g's quads, use(i) scores a slot.  (Past the last whole group a slot
+  // is filled with that again.)
+  auto stream = [&](auto load, auto use) {
+#pragma unroll
+    for (int i = 0; i < PD; ++i) load(i, i, true);
+    int g = 0;
+    for (; g + PD <= nfull; g += PD) {
+#pragma unroll
+      for (int i = 0; i < PD; ++i) use(i, min(g + i + PD, nfull - 1));
+    }
+#pragma unroll
+    for (int i = 0; i < PD - 1; ++i)
+      if (g + i < nfull) use(i, nfull - 1);
+    if (rest) {
+      load(0, nfull, false);
+      use(0, nfull - 1);
+    }
+  };
+
+  Raw rx[PD][PT], rc[PD][CT];
+  auto load_x = [&](int i, int g, bool whole) {
+#pragma unroll
+    for (int p = 0; p < PT; ++p)
+      rx[i][p] = load_quad<DT>(xrow[p], S::FG * g + 4 * q, D, whole);
+  };
+  if (x_sq != nullptr) {
+    given_norms<M, PT>(x_sq + (size_t)b * N, w.n0, N, xs);
+  } else {
+    S::Acc acc[PT];
+#pragma unroll
+    for (int p = 0; p < PT; ++p) acc[p] = S::Acc{0.f, 0.f, 0.f, 0.f};
+    stream(load_x, [&](int i, int next) {
+      Raw u[PT];
+#pragma unroll
+      for (int p = 0; p < PT; ++p) u[p] = rx[i][p];
+      load_x(i, next, true);
+#pragma unroll
+      for (int p = 0; p < PT; ++p) {
+        float v[4];
+        S::steps(Quad<DT>::cvt(u[p]), v);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) acc[p] = S::mfma(v[s], v[s], acc[p]);
+      }
+    });
+#pragma unroll
+    for (int p = 0; p < PT; ++p) xs[p] = diagonal<M>(acc[p]);
+  }
+
   const int nt = (K + M * CT - 1) / (M * CT);
   for (int t = w.kpart; t < nt; t += ks) {
     const int k0 = M * CT * t;
@@ -424,16 +498,19 @@ assign_f32_wide_kernel(const typename Elem<DT>::T* __restrict__ x,
     for (int j = 0; j < CT; ++j)
 #pragma unroll
       for (int p = 0; p < PT; ++p) acc[j][p] = S::Acc{0.f, 0.f, 0.f, 0.f};
-    Raw rx[PT], rc[CT];
-    auto fetch = [&](int g, bool whole) {
-#pragma unroll
-      for (int p = 0; p < PT; ++p)
-        rx[p] = load_quad<DT>(xrow[p], S::FG * g + 4 * q, D, whole);
+    auto load = [&](int i, int g, bool whole) {
+      load_x(i, g, whole);
 #pragma unroll
       for (int j = 0; j < CT; ++j)
-        rc[j] = load_quad<DT>(crow[j], S::FG * g + 4 * q, D, whole);
+        rc[i][j] = load_quad<DT>(crow[j], S::FG * g + 4 * q, D, whole);
     };
-    auto score = [&](const Raw (&ux)[PT], const Raw (&uc)[CT]) {
+    stream(load, [&](int i, int next) {
+      Raw ux[PT], uc[CT];
+#pragma unroll
+      for (int p = 0; p < PT; ++p) ux[p] = rx[i][p];
+#pragma unroll
+      for (int j = 0; j < CT; ++j) uc[j] = rc[i][j];
+      load(i, next, true);
       float a[CT][4], bx[PT][4];
 #pragma unroll
       for (int p = 0; p < PT; ++p) S::steps(Quad<DT>::cvt(ux[p]), bx[p]);
@@ -446,21 +523,7 @@ assign_f32_wide_kernel(const typename Elem<DT>::T* __restrict__ x,
 #pragma unroll
           for (int p = 0; p < PT; ++p)
             acc[j][p] = S::mfma(a[j][s], bx[p][s], acc[j][p]);
-    };
-    fetch(0, true);  // D > 512: group 0 is whole
-    for (int g = 0; g < nfull; ++g) {
-      Raw ux[PT], uc[CT];
-#pragma unroll
-      for (int p = 0; p < PT; ++p) ux[p] = rx[p];
-#pragma unroll
-      for (int j = 0; j < CT; ++j) uc[j] = rc[j];
-      fetch(min(g + 1, nfull - 1), true);
-      score(ux, uc);
-    }
-    if (D % S::FG != 0) {
-      fetch(nfull, false);
-      score(rx, rc);
-    }
+    });
 #pragma unroll
     for (int j = 0; j < CT; ++j) {
       float cq[S::R];
@@ -522,9 +585,9 @@ row_sqnorm_kernel(const typename Elem<DT>::T* __restrict__ src,
 }
 
 // The launch of a shape: instruction shape m, m-point tiles per wave (pt),
-// waves of a workgroup that share their points and split K (ks).
+// 16-centroid tiles at a time (ct: rows above D = 512), waves of a workgroup that share their points and split K (ks).
 struct F32Plan {
-  int m, pt, ks;
+  int m, pt, ct, ks;
 };
 
 // 32 x 32 blocks step eight features at a time, 16 x 16 blocks sixteen: where
@@ -542,7 +605,7 @@ bool f32_has_m32(int64_t D) { return D <= 248 && (D + 7) / 8 % 2 == 1; }
 // one wave alone on a SIMD reaches 0.77 of what two do.
 F32Plan plan_f32(int64_t B, int64_t N, int64_t K, int64_t D) {
   const int64_t simds = 4 * (int64_t)device_shape().cus;
-  F32Plan best{16, 1, 1};
+  F32Plan best{16, 1, 1, 1};
   double least = 0;
   for (int m = 16; m <= 32; m *= 2) {
     if (m == 32 && !f32_has_m32(D)) break;
@@ -559,7 +622,7 @@ F32Plan plan_f32(int64_t B, int64_t N, int64_t K, int64_t D) {
                          groups * ((double)((nt + ks - 1) / ks) * u + 2);
         if (least == 0 || t < least) {
           least = t;
-          best = {m, pt, ks};
+          best = {m, pt, 1, ks};
         }
       }
     }
@@ -567,19 +630,53 @@ F32Plan plan_f32(int64_t B, int64_t N, int64_t K, int64_t D) {
   return best;
 }
 
+// The launch of rows above D = 512: point (1 or 4) and centroid (1, 2 or 4)
+// tiles per wave, waves that split K.  The candidate with the least modelled
+// time: waves per SIMD times a wave's blocks; waves of fewer blocks load more
+// per MFMA (factors that fit the best of all forms at 100 .. 100000 points and
+// 1 .. 1000 centroids; 4 x 1 blocks never were).  Against 4 x 4
+// blocks alone, fp32 us: (1, 1000, 4, 768) 76 -> 11, (1, 20000, 32, 1024) 116
+// -> 47, (1, 100000, 16, 513) 121 -> 65; the vector kernel before them took
+// 18, 86 and 86.
+F32Plan plan_wide(int64_t B, int64_t N, int64_t K) {
+  const int64_t simds = 4 * (int64_t)device_shape().cus;
+  F32Plan best{16, 1, 1, 1};
+  double least = 0;
+  for (int pt = 4; pt >= 1; pt /= 4) {
+    for (int ct = 4; ct >= (pt == 4 ? 2 : 1); ct /= 2) {
+      const int64_t nt = (K + 16 * ct - 1) / (16 * ct);
+      const double reuse = pt == 4 ? (ct == 4 ? 1.0 : 1.2)
+                                   : (ct == 4 ? 1.3 : ct == 2 ? 1.6 : 2.0);
+      for (int ks = 1; ks <= 4 && ks <= nt; ks *= 2) {
+        const int64_t waves = B * ((N + 16 * pt - 1) / (16 * pt)) * ks;
+        const double t = std::max(1.3, (double)waves / (double)simds) * pt *
+                         ct * reuse * (double)((nt + ks - 1) / ks);
+        if (least == 0 || t < least) {
+          least = t;
+          best = {16, pt, ct, ks};
+        }
+      }
+    }
+  }
+  return best;
+}
+
+enum F32Kind { kChain, kWide };
+
+F32Kind f32_kind(int64_t D) { return D > 512 ? kWide : kChain; }
+
+F32Plan f32_plan(F32Kind kind, int64_t B, int64_t N, int64_t K, int64_t D) {
+  if (kind == kWide) return plan_wide(B, N, K);
+  return plan_f32(B, N, K, D);
+}
+
 template <int DT>
 int launch_f32_t(const void* x, const void* c, const float* x_sq,
                  const float* c_sq, int32_t* ids, int64_t B, int64_t N,
                  int64_t K, int64_t D, const int32_t* ctrl, hipStream_t s) {
   using T = typename Elem<DT>::T;
-  F32Plan p{16, 4, 1};
-  if (D <= 512) {
-    p = plan_f32(B, N, K, D);
-  } else {
-    const int64_t want = 8 * (int64_t)device_shape().cus, nt = (K + 63) / 64;
-    while (p.ks < 4 && 2 * p.ks <= nt && B * ((N + 63) / 64) * p.ks < want)
-      p.ks *= 2;
-  }
+  const F32Kind kind = f32_kind(D);
+  const F32Plan p = f32_plan(kind, B, N, K, D);
   const int64_t per = p.m * p.pt * (4 / p.ks);  // points per workgroup
   const dim3 grid((unsigned)((N + per - 1) / per), (unsigned)B);
   auto go = [&](auto kernel) {
@@ -588,7 +685,14 @@ int launch_f32_t(const void* x, const void* c, const float* x_sq,
                        (int)K, (int)D, p.ks, ctrl);
     return check_launch("assign_f32");
   };
-  if (D > 512) return go(assign_f32_wide_kernel<DT>);
+  if (kind == kWide) {
+    if (p.pt == 1)
+      return p.ct == 1   ? go(assign_f32_wide_kernel<DT, 1, 1, 8>)
+             : p.ct == 2 ? go(assign_f32_wide_kernel<DT, 1, 2, 6>)
+                         : go(assign_f32_wide_kernel<DT, 1, 4, 4>);
+    return p.ct == 2 ? go(assign_f32_wide_kernel<DT, 4, 2, 3>)
+                     : go(assign_f32_wide_kernel<DT, 4, 4, 1>);
+  }
   // G feature groups cover D; the NF groups of the next smaller variant are
   // certainly whole (all G where fp32 fills them exactly).  The points'
   // operands take 128 registers at most, which leaves two waves per SIMD.
@@ -689,6 +793,18 @@ int launch_assign(const void* x, const void* c, const float* x_sq,
   }
   if (ev1 != nullptr) (void)hipEventRecord(ev1, s);
   return rc;
+}
+
+void assign_plan(int64_t B, int64_t N, int64_t K, int64_t D, int dtype,
+                 bool slices, int32_t out[6]) {
+  if (assign_uses_mfma(dtype, D)) {
+    assign_mfma_plan(B, N, K, D, slices, out);
+    return;
+  }
+  const F32Kind kind = f32_kind(D);
+  const F32Plan p = f32_plan(kind, B, N, K, D);
+  const int32_t v[6] = {(int32_t)kind, p.m, p.pt, p.ct, p.ks, (int32_t)K};
+  std::copy(v, v + 6, out);
 }
 
 int launch_row_sqnorm(const void* src, float* out, int64_t rows, int64_t D,

@@ -1640,6 +1640,14 @@ size_t assign_workspace_bytes(int64_t B, int64_t N, int64_t K, int64_t D,
                      B, N, nullptr, nullptr);
 }
 
+void assign_mfma_plan(int64_t B, int64_t N, int64_t K, int64_t D, bool slices,
+                      int32_t out[6]) {
+  const Plan p = plan_assign(B, N, K, D, slices);
+  const int kind = p.resident ? 7 : p.whole ? 6 : p.save ? 5 : p.exact ? 3 : 4;
+  const int32_t v[6] = {kind, 16, p.pt, 1, p.S, p.kspan};
+  std::copy(v, v + 6, out);
+}
+
 int launch_assign_mfma(const void* x, const void* c, const float* c_sq,
                        int32_t* ids, int64_t B, int64_t N, int64_t K,
                        int64_t D, int dtype, const int32_t* ctrl,

@@ -354,6 +354,17 @@ int fkc_euclid_assign_ws(const void* x, const void* centroids,
                        nullptr, workspace, workspace_bytes);
 }
 
+int fkc_assign_plan(int64_t B, int64_t N, int64_t K, int64_t D, int dtype,
+                    int slices, int32_t* plan) {
+  g_err[0] = 0;
+  if (int rc = shape_ok(B, N, K, D, "assign_plan")) return rc;
+  if (int rc = dtype_ok(dtype, "assign_plan")) return rc;
+  if (B * N == 0 || !plan)
+    return fail(FKC_ERR_INVALID, "assign_plan: no points or no output");
+  assign_plan(B, N, K, D, dtype, slices != 0, plan);
+  return FKC_OK;
+}
+
 int fkc_row_sqnorm(const void* src, float* out, int64_t rows, int64_t D,
                    int dtype, fkc_stream_t stream) {
   g_err[0] = 0;

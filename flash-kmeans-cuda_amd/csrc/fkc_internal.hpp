@@ -51,6 +51,12 @@ size_t assign_workspace_bytes(int64_t B, int64_t N, int64_t K, int64_t D,
 // ws (optional, assign_workspace_bytes): with it the MFMA route may slice K,
 // with the least one as far as that reaches; without it the launch is never
 // sliced.
+// What launch_assign would launch (fkc_assign_plan's values); slices: with a
+// workspace of assign_workspace_bytes.
+void assign_plan(int64_t B, int64_t N, int64_t K, int64_t D, int dtype,
+                 bool slices, int32_t out[6]);
+void assign_mfma_plan(int64_t B, int64_t N, int64_t K, int64_t D, bool slices,
+                      int32_t out[6]);
 int launch_assign(const void* x, const void* c, const float* x_sq,
                   const float* c_sq, int32_t* ids, int64_t B, int64_t N,
                   int64_t K, int64_t D, int dtype, const int32_t* ctrl,

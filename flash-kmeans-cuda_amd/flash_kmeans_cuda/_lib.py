@@ -56,6 +56,7 @@ SIGNATURES = {
     "fkc_profile_enable": (None, [_int]),
     "fkc_profile_assign_ms": (_int, [ctypes.POINTER(ctypes.c_double), ctypes.POINTER(ctypes.c_int64)]),
     "fkc_kmeans_sort_recounts_offset": (_sz, [_i64, _i64, _i64, _i64, _int, _int]),
+    "fkc_assign_plan": (_int, [_i64, _i64, _i64, _i64, _int, _int, _vp]),
 }
 
 

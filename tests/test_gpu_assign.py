@@ -12,6 +12,8 @@ tests/test_persistent.py:97-165, tests/cpp/smoke.cpp:31-53.
 
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -563,6 +565,85 @@ def test_fp32_route_is_the_fma_chain(B, N, K, D, dtype):
                 v = np.longdouble(xv[:, d])
                 sq = (np.longdouble(sq) + v * v).astype(np.float32)
         assert np.array_equal(own[b, pick], _chain_labels(xv, cv, sq, csb))
+
+
+def _plan(B, N, K, D, dtype):
+    from flash_kmeans_cuda import _lib
+    out = (ctypes.c_int32 * 6)()
+    dt = {"f32": 0, "f16": 1, "bf16": 2}[dtype]
+    assert _lib.lib.fkc_assign_plan(B, N, K, D, dt, 1, out) == 0
+    return tuple(out)
+
+
+@pytest.mark.parametrize("B,N,K,D,dtype,cus", [
+    (1, 3000, 333, 100, "f32", (4, 8, 16, 64, 256)), (2, 2001, 130, 37, "f16", (4, 16, 64, 128, 256)),
+    (1, 1999, 70, 24, "f32", (4, 8, 32, 64, 256)), (1, 777, 33, 200, "f32", (4, 16, 256)),
+    (1, 700, 50, 500, "f32", (4, 32, 256)), (1, 3001, 64, 128, "f32", (4, 8, 64, 128, 256)),
+    (2, 999, 60, 44, "bf16", (4, 8, 32, 64, 256)), (1, 900, 97, 4, "f32", (2, 4, 8, 256)),
+    (1, 2500, 21, 530, "f32", (8, 16, 256)), (1, 2500, 200, 640, "f16", (4, 8, 16, 256)),
+    (1, 4100, 150, 600, "f32", (4, 16, 32, 64, 256)), (3, 1500, 17, 513, "bf16", (8, 32, 256)),
+])
+def test_fp32_plans_agree(monkeypatch, B, N, K, D, dtype, cus):
+    """The fp32 route's block shapes, tiles per wave and K splits, forced by
+    planning for other CU counts: each another plan, with the same labels,
+    those of the chain (equal rows far apart in K, ragged N and K)."""
+    rng = np.random.default_rng(N + K)
+    xf = rng.standard_normal((B, N, D)).astype(np.float32)
+    cf = rng.standard_normal((B, K, D)).astype(np.float32)
+    cf[:, K - 1] = cf[:, 1]
+    xf[:, ::5] = cf[:, [1]]
+    x, c = O.from_f32(xf, dtype), O.from_f32(cf, dtype)
+    plans, got = set(), []
+    for n in cus:
+        monkeypatch.setenv("FKC_CUS", str(n))
+        plans.add(_plan(B, N, K, D, dtype))
+        got += [_gpu_assign(x, c, dtype), _gpu_assign(x, c, dtype, with_xsq=False)]
+    assert len(plans) == len(cus)
+    for g in got[2::2]:
+        assert np.array_equal(got[0], g)
+    for g in got[3::2]:
+        assert np.array_equal(got[1], g)
+    monkeypatch.delenv("FKC_CUS")
+    _check(x, c, dtype, got[0])
+
+
+@pytest.mark.parametrize("B,N,K,D,dtype", [
+    (1, 100, 4, 768, "f32"), (1, 1000, 20, 513, "f16"), (1, 300, 64, 1000, "f32"),
+    (2, 200, 300, 520, "bf16"),
+])
+def test_wide_rows_in_smaller_blocks(B, N, K, D, dtype):
+    assert _plan(B, N, K, D, dtype)[2] == 1
+    test_fp32_route_is_the_fma_chain(B, N, K, D, dtype)
+
+
+def _assign_us(B, N, K, D, given=True):
+    """Best of five timings of fp32 calls, us each."""
+    from flash_kmeans_cuda import _C
+    from flash_kmeans_cuda.ops import row_sqnorm
+    x = torch.randn(B, N, D, device="cuda")
+    c = torch.randn(B, K, D, device="cuda")
+    xs = row_sqnorm(x) if given else torch.empty(0, device="cuda")
+    cs, ids = row_sqnorm(c), torch.empty((B, N), dtype=torch.int32, device="cuda")
+    best = float("inf")
+    for _ in range(6):
+        a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        a.record()
+        for _ in range(20):
+            _C.euclid_assign(x, c, xs, cs, ids)
+        b.record()
+        torch.cuda.synchronize()
+        best = min(best, a.elapsed_time(b) * 50)
+    return best
+
+
+def test_few_points_or_centroids_do_not_wait():
+    """Shapes that once cost a round trip per feature or per group of
+    features.  Ratios between calls, measured before and after: norms in the
+    kernel 5.8 -> 1.0 and 5.3 -> 1.0; rows of 768 against 512 features 8.5 ->
+    1.3."""
+    for shape in ((1, 35, 5, 768), (1, 1000, 4, 768)):
+        assert _assign_us(*shape, given=False) < 2 * _assign_us(*shape)
+    assert _assign_us(1, 1000, 4, 768) < 3 * _assign_us(1, 1000, 4, 512)
 
 
 def test_force_safe_env_routes_to_fp32_kernel(monkeypatch):

@@ -78,23 +78,37 @@ struct Quad<FKC_F32> {
 
 // Features d .. d + 3 of a row of D.  whole: all four exist (d + 3 < D);
 // else those at D and after read as zero, which adds nothing to a chain.
+// Such a quad is the row's last whole one, moved down by the features it
+// starts early: four clamped loads of one feature each took twice the time of
+// whole quads at few features ((1, 400000, 8, D) fp32, us: D = 8 14.5, D = 12
+// 11.4, against 8.1 at D = 16).  Only rows of less than a quad are loaded so.
 template <int DT>
 __device__ inline typename Quad<DT>::Raw load_quad(
-    const typename Elem<DT>::T* row, int d, int D, bool whole) {
+    const typename Elem<DT>::T* row, int d, int D, bool whole, bool tiny) {
   using Raw = typename Quad<DT>::Raw;
   if (whole) return *reinterpret_cast<const Raw*>(row + d);
-  Raw r;
+  Raw r = {};
+  if (tiny) {
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    typename Elem<DT>::T v = row[min(d + e, D - 1)];
-    if constexpr (DT == FKC_F32) {
-      r[e] = d + e < D ? v : 0.f;
-    } else {
-      uint16_t h;
-      __builtin_memcpy(&h, &v, 2);
-      r[e] = d + e < D ? h : (uint16_t)0;
+    for (int e = 0; e < 3; ++e) {
+      const typename Elem<DT>::T v = row[min(d + e, D - 1)];
+      if constexpr (DT == FKC_F32) {
+        r[e] = d + e < D ? v : 0.f;
+      } else {
+        uint16_t h;
+        __builtin_memcpy(&h, &v, 2);
+        r[e] = d + e < D ? h : (uint16_t)0;
+      }
     }
+    return r;
   }
+  const int d0 = min(d, D - 4), early = d - d0;
+  r = *reinterpret_cast<const Raw*>(row + d0);
+  if (D % 4 != 0) {
+    if (early & 1) r = Raw{r[1], r[2], r[3], 0};
+    if (early & 2) r = Raw{r[2], r[3], 0, 0};
+  }
+  if (early > 3) r = Raw{0, 0, 0, 0};
   return r;
 }
 
@@ -331,11 +345,12 @@ assign_f32_kernel(const typename Elem<DT>::T* __restrict__ x,
   const float* qb = c_sq + (size_t)b * K;
 
   const int nt = (K + M - 1) / M;
+  const bool tiny = G == 1 && D < 4;
   // Quad g of this lane's row of tile t (row K - 1 past K: such rows are
   // loaded but never win).
   auto load_c = [&](int t, int g) -> Raw {
     const T* row = cb + (size_t)min(M * t + col, K - 1) * D;
-    return load_quad<DT>(row, S::FG * g + 4 * q, D, g < NF);
+    return load_quad<DT>(row, S::FG * g + 4 * q, D, g < NF, tiny);
   };
   Raw ring[PD];
 #pragma unroll
@@ -348,7 +363,7 @@ assign_f32_kernel(const typename Elem<DT>::T* __restrict__ x,
     Raw raw[G];
 #pragma unroll
     for (int g = 0; g < G; ++g)
-      raw[g] = load_quad<DT>(row, S::FG * g + 4 * q, D, g < NF);
+      raw[g] = load_quad<DT>(row, S::FG * g + 4 * q, D, g < NF, tiny);
 #pragma unroll
     for (int g = 0; g < G; ++g) S::steps(Quad<DT>::cvt(raw[g]), bx[p][g]);
   }
@@ -461,7 +476,7 @@ assign_f32_wide_kernel(const typename Elem<DT>::T* __restrict__ x,
   auto load_x = [&](int i, int g, bool whole) {
 #pragma unroll
     for (int p = 0; p < PT; ++p)
-      rx[i][p] = load_quad<DT>(xrow[p], S::FG * g + 4 * q, D, whole);
+      rx[i][p] = load_quad<DT>(xrow[p], S::FG * g + 4 * q, D, whole, false);
   };
   if (x_sq != nullptr) {
     given_norms<M, PT>(x_sq + (size_t)b * N, w.n0, N, xs);
@@ -502,7 +517,7 @@ assign_f32_wide_kernel(const typename Elem<DT>::T* __restrict__ x,
       load_x(i, g, whole);
 #pragma unroll
       for (int j = 0; j < CT; ++j)
-        rc[i][j] = load_quad<DT>(crow[j], S::FG * g + 4 * q, D, whole);
+        rc[i][j] = load_quad<DT>(crow[j], S::FG * g + 4 * q, D, whole, false);
     };
     stream(load, [&](int i, int next) {
       Raw ux[PT], uc[CT];
@@ -532,6 +547,165 @@ assign_f32_wide_kernel(const typename Elem<DT>::T* __restrict__ x,
     }
   }
   merge_store<M, PT>(best, bidx, ks, w, ids + (size_t)b * N, N);
+}
+
+// The better of two candidates: smaller distance, then smaller index.
+__device__ inline void take_better(float& b, int& i, float ob, int oi) {
+  const bool other = ob < b || (ob == b && oi < i);
+  b = other ? ob : b;
+  i = other ? oi : i;
+}
+
+// Few centroids of few features (K <= 16 KT, D <= 16 G) and many points: the
+// centroids' operands and c_sq stay in registers and a wave walks groups of 64
+// points, the next group's loads in flight.  What bounds it is the vector
+// work per group, so a tile's centroids are laid out with lane group q's
+// register r holding centroid 4 r + q (registers past K are skipped whole),
+// and the four lane groups' winners of four point tiles are merged with lane
+// swaps, each group ending with one tile.  At (1, 3000000, 8, D) fp32, us, the
+// vector kernel (one lane per point), the kernel above, this one: D = 1 28 /
+// 44 / 24, D = 8 33 / 50 / 29, D = 16 40 / 41 / 39 (216 MB: 5.5 TB/s, partly
+// from the cache); D = 24 57 / 70 / 66.
+template <int DT, int G, int KT>
+__global__ void __launch_bounds__(FT, G == 1 ? 4 : 2)
+assign_few_kernel(const typename Elem<DT>::T* __restrict__ x,
+                  const typename Elem<DT>::T* __restrict__ c,
+                  const float* __restrict__ x_sq,
+                  const float* __restrict__ c_sq, int32_t* __restrict__ ids,
+                  int N, int K, int D, const int32_t* __restrict__ ctrl) {
+  using T = typename Elem<DT>::T;
+  using Raw = typename Quad<DT>::Raw;
+  using S = Shape<16>;
+  constexpr int M = 16, PT = 4;
+  if (loop_done(ctrl)) return;
+  const int lane = threadIdx.x & 63, col = lane % M, q = lane / M;
+  const int b = blockIdx.y;
+  const T* xb = x + (size_t)b * N * D;
+  const T* cb = c + (size_t)b * K * D;
+  const float* qb = c_sq + (size_t)b * K;
+  const float* xq = x_sq != nullptr ? x_sq + (size_t)b * N : nullptr;
+  int32_t* ib = ids + (size_t)b * N;
+  const bool tiny = D < 4;
+
+  int n0 = WaveWork(1, M * PT).n0;
+  const int stride = (int)gridDim.x * 4 * M * PT;
+  Raw rx[PT][G];
+  float rq[PT];
+  auto load_x = [&](int at) {
+#pragma unroll
+    for (int p = 0; p < PT; ++p) {
+      const int n = min(at + M * p + col, N - 1);
+      const T* row = xb + (size_t)n * D;
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+        rx[p][g] = load_quad<DT>(row, S::FG * g + 4 * q, D, g < G - 1, tiny);
+      rq[p] = xq != nullptr ? xq[n] : 0.f;
+    }
+  };
+  load_x(n0);
+
+  float a[KT][G][4], cq[KT][S::R];
+#pragma unroll
+  for (int t = 0; t < KT; ++t) {
+    const T* row = cb + (size_t)min(M * t + 4 * (col & 3) + col / 4, K - 1) * D;
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+      S::steps(Quad<DT>::cvt(load_quad<DT>(row, S::FG * g + 4 * q, D,
+                                           g < G - 1, tiny)),
+               a[t][g]);
+#pragma unroll
+    for (int r = 0; r < S::R; ++r) cq[t][r] = qb[min(M * t + 4 * r + q, K - 1)];
+  }
+
+  for (bool more = n0 < N; more; n0 += stride) {
+    more = stride < N - n0;
+    float bx[PT][G][4], xs[PT], best[PT];
+    int bidx[PT];
+#pragma unroll
+    for (int p = 0; p < PT; ++p) {
+#pragma unroll
+      for (int g = 0; g < G; ++g) S::steps(Quad<DT>::cvt(rx[p][g]), bx[p][g]);
+      xs[p] = rq[p];
+    }
+    if (more) load_x(n0 + stride);
+    if (xq == nullptr) {
+#pragma unroll
+      for (int p = 0; p < PT; ++p) {
+        S::Acc acc = {};
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+#pragma unroll
+          for (int s = 0; s < 4; ++s)
+            if (S::FG * g + 4 * s < D)
+              acc = S::mfma(bx[p][g][s], bx[p][g][s], acc);
+        xs[p] = diagonal<M>(acc);
+      }
+    }
+#pragma unroll
+    for (int p = 0; p < PT; ++p) {
+      best[p] = FLT_MAX;
+      bidx[p] = 0;
+    }
+#pragma unroll
+    for (int t = 0; t < KT; ++t) {
+      S::Acc acc[PT];
+#pragma unroll
+      for (int p = 0; p < PT; ++p) acc[p] = S::Acc{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+          if (S::FG * g + 4 * s < D) {
+#pragma unroll
+            for (int p = 0; p < PT; ++p)
+              acc[p] = S::mfma(a[t][g][s], bx[p][g][s], acc[p]);
+          }
+      // As fold_dist; centroid k0 + q, the last register's past K masked.
+      auto fold = [&](int r, bool whole) {
+        const int k0 = M * t + 4 * r;
+#pragma unroll
+        for (int p = 0; p < PT; ++p) {
+          const float dist = fmaf(-2.0f, acc[p][r], xs[p] + cq[t][r]);
+          float nb = __builtin_amdgcn_fmed3f(dist, 0.f, best[p]);
+          if (!whole) nb = k0 + q < K ? nb : best[p];
+          bidx[p] = nb < best[p] ? k0 : bidx[p];
+          best[p] = nb;
+        }
+      };
+#pragma unroll
+      for (int r = 0; r < S::R; ++r) {
+        if (M * t + 4 * r + 4 <= K)
+          fold(r, true);
+        else if (M * t + 4 * r < K)
+          fold(r, false);
+      }
+    }
+    // No score below FLT_MAX: index 0, as the scan starts.
+#pragma unroll
+    for (int p = 0; p < PT; ++p) bidx[p] = best[p] < FLT_MAX ? bidx[p] + q : 0;
+    // Tiles 0 | 2 and 1 | 3 over the halves of the wave, then even | odd tiles
+    // over the halves' halves: lane group q keeps tile q.
+    float bv[2];
+    int bi[2];
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      const u32x2 v = __builtin_amdgcn_permlane32_swap(
+          __float_as_uint(best[p]), __float_as_uint(best[p + 2]), false, false);
+      const u32x2 i = __builtin_amdgcn_permlane32_swap(
+          (unsigned)bidx[p], (unsigned)bidx[p + 2], false, false);
+      bv[p] = __uint_as_float(v[0]);
+      bi[p] = (int)i[0];
+      take_better(bv[p], bi[p], __uint_as_float(v[1]), (int)i[1]);
+    }
+    const u32x2 v = __builtin_amdgcn_permlane16_swap(
+        __float_as_uint(bv[0]), __float_as_uint(bv[1]), false, false);
+    const u32x2 i = __builtin_amdgcn_permlane16_swap((unsigned)bi[0],
+                                                     (unsigned)bi[1], false, false);
+    float win = __uint_as_float(v[0]);
+    int id = (int)i[0];
+    take_better(win, id, __uint_as_float(v[1]), (int)i[1]);
+    if (lane < N - n0) ib[n0 + lane] = id;
+  }
 }
 
 // Bound by HBM at many rows.  R rows per wave, their loads in flight together:
@@ -585,7 +759,8 @@ row_sqnorm_kernel(const typename Elem<DT>::T* __restrict__ src,
 }
 
 // The launch of a shape: instruction shape m, m-point tiles per wave (pt),
-// 16-centroid tiles at a time (ct: rows above D = 512), waves of a workgroup that share their points and split K (ks).
+// 16-centroid tiles at a time (ct: rows above D = 512, and the few-centroid
+// kernel's KT), waves of a workgroup that share their points and split K (ks).
 struct F32Plan {
   int m, pt, ct, ks;
 };
@@ -598,6 +773,9 @@ struct F32Plan {
 // 426) and wastes less of a small K.
 bool f32_has_m32(int64_t D) { return D <= 248 && (D + 7) / 8 % 2 == 1; }
 
+// 32 x 32 blocks need more than 16 centroids: (1, 1500000, 16, 24) fp32 67 us,
+// with 16 x 16 blocks 33.
+//
 // The candidate with the least modelled time: waves per SIMD, rounded up,
 // times a wave's work in 16 x 16 blocks.  A wave's own start costs about two
 // 16-centroid tiles; fewer points per wave mean more centroid loads per MFMA
@@ -608,7 +786,7 @@ F32Plan plan_f32(int64_t B, int64_t N, int64_t K, int64_t D) {
   F32Plan best{16, 1, 1, 1};
   double least = 0;
   for (int m = 16; m <= 32; m *= 2) {
-    if (m == 32 && !f32_has_m32(D)) break;
+    if (m == 32 && (!f32_has_m32(D) || K <= 16)) break;
     const int u = m / 16;
     const int64_t nt = (K + m - 1) / m;
     const double groups = m == 16 ? 2 * ((D + 15) / 16) : (D + 7) / 8;
@@ -628,6 +806,17 @@ F32Plan plan_f32(int64_t B, int64_t N, int64_t K, int64_t D) {
     }
   }
   return best;
+}
+
+// Where assign_few_kernel is taken: its registers hold the centroids, and
+// there are enough points for its waves to walk.  At (1, N, K, D) fp32, us,
+// assign_f32_kernel / this: N = 500000: (16, 16) 10 / 10, (48, 16) 16 / 16,
+// (16, 24) 15 / 14, (48, 8) 14 / 12; N = 3000000: (16, 16) 41 / 40, (48, 16)
+// 73 / 73, (16, 24) 70 / 67, (16, 28) 75 / 77, (32, 20) 68 / 78, (32, 8) 46 /
+// 45, (17, 1) 47 / 36; below 131072 points both end before the next launch.
+bool f32_few(int64_t B, int64_t N, int64_t K, int64_t D) {
+  return ((D <= 16 && K <= 48) || (D <= 24 && K <= 16)) && N >= 1024 &&
+         B * N >= 131072;
 }
 
 // The launch of rows above D = 512: point (1 or 4) and centroid (1, 2 or 4)
@@ -661,12 +850,15 @@ F32Plan plan_wide(int64_t B, int64_t N, int64_t K) {
   return best;
 }
 
-enum F32Kind { kChain, kWide };
+enum F32Kind { kChain, kWide, kFew };
 
-F32Kind f32_kind(int64_t D) { return D > 512 ? kWide : kChain; }
+F32Kind f32_kind(int64_t B, int64_t N, int64_t K, int64_t D) {
+  return D > 512 ? kWide : f32_few(B, N, K, D) ? kFew : kChain;
+}
 
 F32Plan f32_plan(F32Kind kind, int64_t B, int64_t N, int64_t K, int64_t D) {
   if (kind == kWide) return plan_wide(B, N, K);
+  if (kind == kFew) return {16, 4, D > 16 || K <= 16 ? 1 : K <= 32 ? 2 : 3, 1};
   return plan_f32(B, N, K, D);
 }
 
@@ -675,10 +867,27 @@ int launch_f32_t(const void* x, const void* c, const float* x_sq,
                  const float* c_sq, int32_t* ids, int64_t B, int64_t N,
                  int64_t K, int64_t D, const int32_t* ctrl, hipStream_t s) {
   using T = typename Elem<DT>::T;
-  const F32Kind kind = f32_kind(D);
+  const F32Kind kind = f32_kind(B, N, K, D);
   const F32Plan p = f32_plan(kind, B, N, K, D);
   const int64_t per = p.m * p.pt * (4 / p.ks);  // points per workgroup
-  const dim3 grid((unsigned)((N + per - 1) / per), (unsigned)B);
+  dim3 grid((unsigned)((N + per - 1) / per), (unsigned)B);
+  if (kind == kFew) {
+    // One round of resident workgroups (4 per CU), or two of 6 for the
+    // smallest: us at 3, 4, 6, 8, 12 per CU, (1, 3000000, 8, 8) 41 / 34 / 28 /
+    // 34 / 29, (1, 3000000, 24, 8) 51 / 44 / 53 / 45 / 46.
+    const int64_t most = (D <= 16 && K <= 16 ? 12 : 4) * device_shape().cus;
+    grid.x = (unsigned)std::min<int64_t>(grid.x, std::max<int64_t>(most / B, 1));
+    auto few = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, grid, dim3(FT), 0, s,
+                         static_cast<const T*>(x), static_cast<const T*>(c),
+                         x_sq, c_sq, ids, (int)N, (int)K, (int)D, ctrl);
+      return check_launch("assign_few");
+    };
+    return D > 16      ? few(assign_few_kernel<DT, 2, 1>)
+           : p.ct == 1 ? few(assign_few_kernel<DT, 1, 1>)
+           : p.ct == 2 ? few(assign_few_kernel<DT, 1, 2>)
+                       : few(assign_few_kernel<DT, 1, 3>);
+  }
   auto go = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, grid, dim3(FT), 0, s, static_cast<const T*>(x),
                        static_cast<const T*>(c), x_sq, c_sq, ids, (int)N,
@@ -801,7 +1010,7 @@ void assign_plan(int64_t B, int64_t N, int64_t K, int64_t D, int dtype,
     assign_mfma_plan(B, N, K, D, slices, out);
     return;
   }
-  const F32Kind kind = f32_kind(D);
+  const F32Kind kind = f32_kind(B, N, K, D);
   const F32Plan p = f32_plan(kind, B, N, K, D);
   const int32_t v[6] = {(int32_t)kind, p.m, p.pt, p.ct, p.ks, (int32_t)K};
   std::copy(v, v + 6, out);

@@ -608,6 +608,24 @@ def test_fp32_plans_agree(monkeypatch, B, N, K, D, dtype, cus):
 
 
 @pytest.mark.parametrize("B,N,K,D,dtype", [
+    # register rows of centroids and quads of features partly used, one to
+    # three centroid tiles, 16 features filled and passed, several points
+    # groups per wave and a ragged last one, batches
+    (1, 131073, 1, 1, "f32"), (2, 70001, 5, 3, "f32"), (1, 140000, 16, 16, "f32"),
+    (1, 140000, 17, 8, "f32"), (1, 140000, 33, 13, "f32"), (1, 140000, 48, 12, "f32"),
+    (1, 140000, 16, 24, "f32"), (4, 70000, 3, 17, "f32"), (1, 262145, 20, 5, "f16"),
+    (1, 140000, 47, 15, "bf16"), (3, 50000, 4, 20, "bf16"),
+])
+@pytest.mark.parametrize("cus", ["16", "256"])
+def test_few_centroids_of_few_features(monkeypatch, cus, B, N, K, D, dtype):
+    """The kernel that keeps the centroids in registers, bit for bit the
+    chain, with one and with many groups of points per wave."""
+    monkeypatch.setenv("FKC_CUS", cus)
+    assert _plan(B, N, K, D, dtype)[0] == 2
+    test_fp32_route_is_the_fma_chain(B, N, K, D, dtype)
+
+
+@pytest.mark.parametrize("B,N,K,D,dtype", [
     (1, 100, 4, 768, "f32"), (1, 1000, 20, 513, "f16"), (1, 300, 64, 1000, "f32"),
     (2, 200, 300, 520, "bf16"),
 ])
@@ -640,10 +658,11 @@ def test_few_points_or_centroids_do_not_wait():
     """Shapes that once cost a round trip per feature or per group of
     features.  Ratios between calls, measured before and after: norms in the
     kernel 5.8 -> 1.0 and 5.3 -> 1.0; rows of 768 against 512 features 8.5 ->
-    1.3."""
+    1.3; rows of 8 against 16 features, many points, 1.3 -> 0.75."""
     for shape in ((1, 35, 5, 768), (1, 1000, 4, 768)):
         assert _assign_us(*shape, given=False) < 2 * _assign_us(*shape)
     assert _assign_us(1, 1000, 4, 768) < 3 * _assign_us(1, 1000, 4, 512)
+    assert _assign_us(1, 3000000, 1, 8) < 1.1 * _assign_us(1, 3000000, 1, 16)
 
 
 def test_force_safe_env_routes_to_fp32_kernel(monkeypatch):

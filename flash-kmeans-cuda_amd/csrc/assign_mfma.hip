@@ -1293,20 +1293,8 @@ bool assign_uses_mfma(int dtype, int64_t D) {
 // (measured on MI355X's 256 CUs at N = 131072, K = 2048 and N = 65536,
 // K = 8192: four tiles on 512 / 256 workgroups beat two tiles on 1024 / 512
 // by 3% / 5%); eight tiles run 2 workgroups per CU and need two rounds of
-// them.  Wide rows (D > 128) are bound by their LDS fragment reads: at
-// D = 256 two tiles read 128 bytes a cycle from LDS to keep the matrix cores
-// busy, all a CU has, four tiles half of it, so more tiles pay on fewer
-// workgroups.  Same-box fp16 assign times (us), tiles per wave 1 / 2 / 4:
-//   (49152, 2000, 160) 54 / 51 / 56      (49152, 2000, 256) 81 / 67 / 79
-//   (32768, 2000, 256) 50 / 49 / 78      (32768, 300, 256) 11 / 13 / 19
-//   (100000, 4096, 256) 302 / 245 / 224  (65536, 2048, 256) 96 / 74 / 80
-//   (262144, 2048, 256) 361 / 275 / 239  (262144, 2048, 160) 271 / 187 / 166
-// and 1 / 2 above D = 256, where one tile also runs one workgroup per CU:
-//   (16384, 2000, 512) 77 / 109          (24000, 2000, 512) 150 / 111
-//   (131072, 2048, 512) 602 / 289        (262144, 2048, 320) 783 / 379.
+// them.  (D <= 128; wider rows: wide_model.)
 static int64_t fill_wgs(int pt, int ds2, bool exact, int64_t cus) {
-  if (ds2 >= 9 && pt == 2) return cus / 2 + 1;
-  if (ds2 >= 5 && pt >= 2) return cus + cus / 2;
   return (!exact && pt == 4 && ds2 == 4) ? cus : 4 * cus;
 }
 
@@ -1314,13 +1302,61 @@ static int64_t grid_wgs(int pt, int64_t B, int64_t N) {
   return B * ((N + 64 * pt - 1) / (64 * pt));
 }
 
+// Modelled time (us, without the launch) of a launch of rows above D = 128:
+// wgs workgroups of pt tiles that score span rows each, in S slices.
+//
+// These launches run in rounds of one to three workgroups per CU, so what
+// decides between one, two and four tiles per wave is the busiest CU's share:
+// its time for one workgroup, for two (side by side where registers and LDS
+// hold two), and for each one more (0: two by two).  In ns per centroid row
+// and 32 features, a re-score counted as 650 rows (exact index: 1.3 times as
+// much per row, 100 rows); fitted to fp16 launches of 16384 .. 524288 points,
+// K = 16 .. 4096, D = 136 .. 512, the chosen tiles within 0.4% of the best of
+// the three on average and 8% at worst.  Few rows per point are bound by the
+// points' loads (load, ns per tile and 32 features).  Same-box fp16 us, tiles
+// per wave 1 / 2 / 4:
+//   (40000, 2000, 256) 82 / 67 / 81      (65536, 2048, 256) 99 / 77 / 82
+//   (150000, 512, 160) 52 / 40 / 46      (262144, 512, 160) 81 / 60 / 54
+//   (150000, 2048, 192) 217 / 143 / 158  (262144, 2048, 160) 290 / 190 / 164
+//   (400000, 64, 160) 28 / 23 / 26       (24000, 1000, 264) 38 / 47
+//   (131072, 2048, 320) 402 / 200        (80000, 512, 264) 52 / 34.
+static double wide_model(int ds2, int pt, bool exact, int64_t wgs, int64_t span,
+                         int64_t S, int64_t cus) {
+  struct Cost {
+    double one, two, more, load;
+  };
+  // Up to D = 192, 224, 256, 288 and 512, for 1, 2, 4 tiles.
+  static const Cost cost[5][3] = {
+      {{2.2, 2.96, 1.29, 200}, {3.0, 3.9, 1.76, 175}, {4.3, 5.9, 0, 195}},
+      {{2.04, 2.65, 0, 200}, {2.58, 3.5, 0, 190}, {3.9, 5.6, 0, 175}},
+      {{1.69, 2.18, 0, 170}, {2.25, 3.2, 0, 166}, {3.85, 5.46, 0, 172}},
+      {{1.98, 2.6, 0, 170}, {3.43, 3.93, 0, 170}, {}},
+      {{1.77, 3.54, 1.77, 170}, {2.63, 3.4, 0, 170}, {}}};
+  const int w = ds2 <= 6 ? 0 : ds2 <= 9 ? ds2 - 6 : 4;
+  Cost c = cost[w][pt == 1 ? 0 : pt == 2 ? 1 : 2];
+  if (exact && ds2 == 9 && pt == 2) {
+    c = {3.24, 3.77, 1.56, 170};  // here three workgroups fit a CU
+  } else if (exact) {
+    c.one *= 1.2;
+    c.two *= 1.06;
+  }
+  const int64_t r = (wgs + cus - 1) / cus;
+  const double share = r == 1   ? c.one
+                       : r == 2 ? c.two
+                       : c.more > 0 ? (double)r * c.more
+                                    : (double)(r / 2) * c.two + (double)(r % 2) * c.one;
+  const double rows = exact ? 1.3 * ((double)span + 100) : (double)span + 650;
+  return std::max(share * rows, (double)r * pt * c.load) * ds2 * 1e-3 +
+         (S > 1 ? 3.0 + 0.03 * (double)S : 0.0);
+}
+
 static bool pt8_ok(int ds2, bool pad, bool exact) {
   return ds2 == 4 && !pad && !exact;
 }
 
-// Tiles per wave for an unsliced launch: the largest of 8 (unpadded
-// D = 128, re-score epilogue only), 4, 2, 1 (bounded by the 64-VGPR point
-// budget) whose grid fills the chip (fill_wgs); fewer, fatter workgroups
+// Tiles per wave for an unsliced launch: above D = 128 what wide_model finds
+// fastest, else the largest of 8 (unpadded D = 128, re-score epilogue only),
+// 4, 2, 1 whose grid fills the chip (fill_wgs); fewer, fatter workgroups
 // reuse each LDS centroid stage more, but grids that leave CUs idle hide
 // latency badly (measured at the c2..c5 shapes; eight tiles at D = 64 ran
 // slower than four).  From K = 8192 one full round of eight-tile
@@ -1335,10 +1371,21 @@ static int choose_pt(int ds2, bool pad, bool exact, int64_t B, int64_t N,
   const int o = ntiles_override();
   if (o == 8 && pt8_ok(ds2, pad, exact)) return o;
   if (o != 0 && o != 8 && (o * ds2 * 4 <= 64 || wide_pt(ds2, o))) return o;
+  if (ds2 > 4) {
+    int best = 2;
+    double least = wide_model(ds2, 2, exact, grid_wgs(2, B, N), K, 1, cus);
+    for (int pt : {1, 4}) {
+      if (pt == 4 && !wide_pt(ds2, 4)) continue;
+      const double t = wide_model(ds2, pt, exact, grid_wgs(pt, B, N), K, 1, cus);
+      if (t < least) {
+        least = t;
+        best = pt;
+      }
+    }
+    return best;
+  }
   for (int pt = 8; pt > 1; pt >>= 1) {
-    if (pt == 8 ? !pt8_ok(ds2, pad, exact)
-                : pt * ds2 * 4 > 64 && !wide_pt(ds2, pt))
-      continue;
+    if (pt == 8 && !pt8_ok(ds2, pad, exact)) continue;
     if (grid_wgs(pt, B, N) >= fill_wgs(pt, ds2, exact, cus)) return pt;
     if (pt == 8 && K >= 8192 && grid_wgs(8, B, N) >= 2 * cus)
       return 8;
@@ -1432,6 +1479,41 @@ static bool keep_small(const Plan& p, int64_t B, int64_t N, int64_t K,
   return (nt == 0 || nt == 4) && save_override() != 0 && resident_override() != 1;
 }
 
+// Above D = 128 wide_model chooses among the tiles per wave and up to `most`
+// slices, against the plan given (bar: the share of its time to get below; in
+// 462 launches of 1000 .. 100000 points the choice took 0.8% more than the
+// best of 1 .. 16 slices).  fp16 us: (24000, 4096, 264) two tiles unsliced 158,
+// one on two slices 109, two on two 99; (49152, 4096, 136) two tiles unsliced
+// 92, on two slices 72; (100000, 4096, 256) two tiles on two slices 241, four
+// unsliced 188.
+static Plan wide_slices(const Plan& p, int64_t B, int64_t N, int64_t K,
+                        int64_t most, double bar, int64_t cus) {
+  Plan best = p;
+  double least = bar * wide_model(p.ds2, p.pt, false, grid_wgs(p.pt, B, N) * p.S,
+                                  p.kspan, p.S, cus);
+  for (int pt : {2, 1, 4}) {
+    if (pt == 4 && !wide_pt(p.ds2, 4)) continue;
+    const int64_t tiles = grid_wgs(pt, B, N);
+    for (int64_t per = 1; per <= 4; ++per) {  // workgroups per CU
+      const int64_t want =
+          std::min(std::max<int64_t>(per * cus / tiles, 2), most);
+      const int64_t span = ((K + want - 1) / want + 127) / 128 * 128;
+      const int64_t S = (K + span - 1) / span;
+      if (S <= 1) continue;
+      // (One tile per wave has to be 4% better: it reads the most centroids.)
+      const double t = wide_model(p.ds2, pt, false, tiles * S, span, S, cus) *
+                       (pt == 1 ? 1.04 : 1.0);
+      if (t < least) {
+        least = t;
+        best.pt = pt;
+        best.S = (int)S;
+        best.kspan = (int)span;
+      }
+    }
+  }
+  return best;
+}
+
 // Launch plan.  K is sliced only when no unsliced grid fills the chip (few
 // points, many centroids): the most tiles the point budget allows (four up
 // to D = 128) then run on S slices of kspan rows
@@ -1442,7 +1524,8 @@ static bool keep_small(const Plan& p, int64_t B, int64_t N, int64_t K,
 // against 0.073 ms unsliced; at N = 80000, K = 70000, D = 16 four slices
 // took 0.376 ms against 0.756 ms, and at N = 8192, K = 65536, D = 128
 // eight slices 0.150 ms against 0.531 ms.  At D = 97..128 the slices fill
-// one round of resident workgroups (below).  FKC_KSPLIT forces S.
+// one round of resident workgroups (below), above D = 128 wide_model decides
+// (wide_slices).  FKC_KSPLIT forces S.
 static Plan plan_filled(int64_t B, int64_t N, int64_t K, int64_t D,
                         bool can_slice, const DeviceShape& dev) {
   const int64_t cus = dev.cus;
@@ -1489,7 +1572,18 @@ static Plan plan_filled(int64_t B, int64_t N, int64_t K, int64_t D,
   // workgroups beat eight on 512 (N = 8192, K = 65536: 0.150 vs 0.166 ms;
   // N = 16384, K = 32768: 0.142 vs 0.156 ms).
   int pt = p.pt;
-  if (ntiles_override() == 0) pt = p.ds2 <= 4 ? 4 : 2;
+  if (ntiles_override() == 0) {
+    if (p.ds2 > 4 && ksplit_override() == 0) {
+      // No more slices than give two tiles (one above D = 256) four
+      // workgroups per CU, which is what callers size their workspaces for.
+      const int64_t t = grid_wgs(p.ds2 <= 8 ? 2 : 1, B, N);
+      int64_t most = 1;
+      while (t * most < 4 * cus && K / (2 * most) >= FKC_SLICE_MIN_ROWS)
+        most *= 2;
+      return wide_slices(p, B, N, K, most, 1.0, cus);
+    }
+    pt = p.ds2 <= 4 ? 4 : 2;
+  }
   int64_t tiles = grid_wgs(pt, B, N);
   int64_t S = ksplit_override();
   if (S == 0 && pt == 4 && p.ds2 == 4) {
@@ -1518,21 +1612,10 @@ static Plan plan_filled(int64_t B, int64_t N, int64_t K, int64_t D,
     }
     if (S <= 1) return p;
   } else if (S == 0) {
-    // (Above D = 256 one tile per wave runs one workgroup per CU; two tiles
-    // run two, and beat it wherever their grid passes fill_wgs: (16384,
-    // 8192, 320) fp16 220 -> 102 us, but (1799, 16610, 408) 75 -> 106.)
-    for (;;) {
-      const int64_t want = (wide_pt(p.ds2, pt) ? 2 : 4) * cus;
-      tiles = grid_wgs(pt, B, N);
-      if (tiles >= want) return p;
-      S = 1;
-      while (tiles * S < want && K / (2 * S) >= FKC_SLICE_MIN_ROWS) S *= 2;
-      if (ntiles_override() != 0 || !wide_pt(p.ds2, pt) ||
-          tiles * S >= fill_wgs(pt, p.ds2, p.exact, cus))
-        break;
-      pt = 1;
-    }
-    const int64_t want = (wide_pt(p.ds2, pt) ? 2 : 4) * cus;
+    const int64_t want = fill_wgs(pt, p.ds2, p.exact, cus);
+    if (tiles >= want) return p;
+    S = 1;
+    while (tiles * S < want && K / (2 * S) >= FKC_SLICE_MIN_ROWS) S *= 2;
     // Slices that still leave the chip short only pay off when the unsliced
     // grid is short too.
     if (tiles * S < want &&
@@ -1587,14 +1670,16 @@ static Plan plan_assign(int64_t B, int64_t N, int64_t K, int64_t D,
     return p;
   const int64_t cus = dev.cus;
   const int64_t old_wgs = grid_wgs(p.pt, B, N) * p.S;
-  const double old = grid_model(p, old_wgs, cus);
+  const double old = p.ds2 > 4 ? wide_model(p.ds2, p.pt, false, old_wgs, p.kspan,
+                                            p.S, cus)
+                               : grid_model(p, old_wgs, cus);
   if (old_wgs >= 2 * cus || old < 17.0 || ksplit_override() != 0 ||
       ntiles_override() != 0)
     return p;
+  if (p.ds2 > 4) return wide_slices(p, B, N, K, K / 128, 0.85, cus);
   Plan best = p;
   double least = 0.78 * old;
   for (int pt = 4; pt >= 1; pt >>= 1) {
-    if (pt * p.ds2 * 4 > 64) continue;
     const int64_t tiles = grid_wgs(pt, B, N);
     for (int64_t per = 1; per <= 3; ++per) {  // workgroups per CU
       const int64_t want = std::min<int64_t>(per * cus / tiles, K / 128);

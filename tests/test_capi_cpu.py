@@ -207,6 +207,52 @@ def test_assign_asks_for_whole_slices_only(monkeypatch, B, N, K, D, nbytes):
                                   nbytes - 1, None) == 2
 
 
+def _plan(B, N, K, D, dtype, slices):
+    from flash_kmeans_cuda import _lib
+    out = (ctypes.c_int32 * 6)()
+    assert _lib.lib.fkc_assign_plan(B, N, K, D, dtype, slices, out) == 0
+    return tuple(out)
+
+
+@pytest.mark.parametrize("N,K,D,tiles", [
+    # Shapes where more tiles per wave leave a last round of workgroups nearly
+    # empty (two tiles, or one, were 10 to 20% faster than four, or two) ...
+    (150000, 512, 160, 2), (150000, 2048, 192, 2), (200000, 64, 160, 2), (400000, 128, 136, 2),
+    (150000, 300, 192, 2), (24000, 1000, 264, 1), (24000, 300, 264, 1), (80000, 1000, 264, 1),
+    # ... and where they fill it.
+    (262144, 512, 160, 4), (262144, 2048, 256, 4), (524288, 1000, 192, 4), (131072, 2048, 512, 2),
+    (80000, 512, 264, 2), (65536, 512, 256, 2), (16384, 1000, 512, 1),
+])
+def test_tiles_of_wide_rows_fit_the_rounds(monkeypatch, N, K, D, tiles):
+    """MI355X plans of unsliced 16-bit assigns above D = 128."""
+    for v in ("FKC_NTILES", "FKC_KSPLIT"):
+        monkeypatch.delenv(v, raising=False)
+    monkeypatch.setenv("FKC_CUS", "256")
+    assert _plan(1, N, K, D, 1, 0)[2] == tiles
+
+
+def test_slices_of_wide_rows(monkeypatch):
+    """Whole slices where they beat an unsliced grid, more tiles where those
+    do; never more than two tiles (one above D = 256) need."""
+    for v in ("FKC_NTILES", "FKC_KSPLIT"):
+        monkeypatch.delenv(v, raising=False)
+    monkeypatch.setenv("FKC_CUS", "256")
+    assert _plan(1, 24000, 4096, 264, 1, 1)[2:] == (2, 1, 2, 2048)
+    assert _plan(1, 49152, 4096, 136, 1, 1)[2:] == (2, 1, 2, 2048)
+    assert _plan(1, 100000, 4096, 256, 1, 1)[2:] == (4, 1, 1, 4096)
+    from flash_kmeans_cuda import _lib
+    need = _lib.lib.fkc_euclid_assign_workspace_bytes
+    for D in (136, 192, 256, 264, 384, 512):
+        for N in (700, 5000, 20000, 60000, 120000):
+            for K in (4096, 9000, 30000):
+                tiles = -(-N // (64 * (2 if D <= 256 else 1)))
+                S = 1
+                while tiles * S < 1024 and K // (2 * S) >= 2048:
+                    S *= 2
+                half = (S * N * 4 + 255) // 256 * 256
+                assert need(1, N, K, D, 1) <= (2 * half if S > 1 else 0), (N, K, D)
+
+
 def test_workspace_sizes():
     from flash_kmeans_cuda import _lib
     L = _lib.lib

@@ -1459,22 +1459,33 @@ static bool use_resident(const Plan& p, int64_t B, int64_t N, int64_t K,
 }
 
 // At K <= FKC_EXACT_MAX_K the exact in-loop index costs 13 vector instructions
-// per four scores against the kept scores' 8, and its loop is not pipelined;
-// it wins only on tables too short to amortise the kept scores' 128-row
-// stages and on small grids.  Same-box bf16 assign times (us), exact index
-// against kept scores with four tiles: D = 128, K = 512: N = 40000 13.0 /
-// 12.1, 65536 15.2 / 12.2, 100000 24.5 / 17.2, 131072 20.0 / 17.8, 262144
-// 43.2 / 34.1, 524288 70.6 / 61.3; K = 256: 40000 8.4 / 8.6, 65536 9.8 / 8.6,
-// 524288 43.3 / 39.0; K = 128: 200000 15.3 / 15.5; K = 64: 262144 15.1 / 17.2.
-// D = 64, K = 512: 200000 22.2 / 20.6, 1000000 73.3 / 62.3; K = 384: 262144
-// 18.5 / 18.4; K = 256: 262144 14.7 / 15.7.
+// per four scores against the kept scores' 8, and its loop is not pipelined.
+// But at D = 128 it stages 64 rows where the kept scores stage 128, so a K that
+// ends in the first half of such a stage is left to it unless its grid only
+// fills with one tile per wave; and where it fills with four, a last round of
+// kept-score workgroups (2 per CU) must be nearly full too.  Same-box fp16
+// assign times (us), exact index / kept scores with four tiles, D = 128:
+//   K       N = 65536     100000       131072       262144       500000     981512
+//   192     8.4 / 8.9   13.1 / 13.2  11.8 / 13.3  23.6 / 25.4  37.4 / 43.6  64 / 77
+//   256     9.7 / 9.0   15.6 / 13.3  13.7 / 13.4  27.6 / 25.7  43.9 / 43.6  78 / 77
+//   320    11.0 / 10.9  18.1 / 16.0  15.9 / 16.2  32.6 / 32.4  51.8 / 57.7  90 / 109
+//   384    12.3 / 10.9  20.3 / 16.0  17.6 / 16.3  36.1 / 32.7  58.3 / 58.8 103 / 109
+//   448    13.7 / 12.6  23.0 / 19.1  19.6 / 19.7  41.0 / 38.4  67.3 / 69.9 118 / 129
+//   512    15.2 / 12.5  25.3 / 19.1  21.8 / 19.8  45.0 / 38.4  73.3 / 68.9 127 / 129.
+// At D = 64 both stage 128 rows: K = 384 19.3 / 20.2 at N = 262144, 35.8 / 37.5
+// at 500000; K = 512 23.9 / 23.3, 43.8 / 41.4, and 79.0 / 74.4 at 981512.
 static bool keep_small(const Plan& p, int64_t B, int64_t N, int64_t K,
                        int64_t cus) {
-  if (p.pad || K > FKC_EXACT_MAX_K || K <= (p.ds2 == 4 ? 128 : 256) ||
+  if (p.pad || K > FKC_EXACT_MAX_K || K <= (p.ds2 == 4 ? 128 : 384) ||
       (p.ds2 != 4 && p.ds2 != 2))
     return false;
   const int64_t wgs = grid_wgs(4, B, N);
   if (p.ds2 == 4 ? 4 * wgs < 3 * cus : wgs < 3 * cus) return false;
+  if (p.ds2 == 4) {
+    const bool half = (K + 63) / 64 % 2 == 1;
+    if (half && (p.pt > 1 || K <= 256)) return false;
+    if (p.pt == 4 && round_fill(wgs, 2 * cus) < 0.95) return false;
+  }
   const int nt = ntiles_override();
   return (nt == 0 || nt == 4) && save_override() != 0 && resident_override() != 1;
 }

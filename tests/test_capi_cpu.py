@@ -253,6 +253,23 @@ def test_slices_of_wide_rows(monkeypatch):
                 assert need(1, N, K, D, 1) <= (2 * half if S > 1 else 0), (N, K, D)
 
 
+@pytest.mark.parametrize("N,K,D,kept", [
+    # D = 128: where the last 128-row stage is at most half used, the exact
+    # index's 64-row stages were up to 23% faster ...
+    (131072, 192, 128, False), (500000, 129, 128, False), (981512, 271, 128, False),
+    (500000, 320, 128, False), (981512, 400, 128, False), (981512, 384, 128, False),
+    # ... and the kept scores where it is used, or the grid is short of points.
+    (131072, 256, 128, True), (100000, 300, 128, True), (500000, 512, 128, True),
+    (262144, 384, 128, True), (65536, 448, 128, True),
+    (500000, 300, 64, False), (262144, 384, 64, False), (500000, 512, 64, True),
+])
+def test_kept_scores_at_small_k_only_where_faster(monkeypatch, N, K, D, kept):
+    for v in ("FKC_NTILES", "FKC_SAVE", "FKC_RESIDENT"):
+        monkeypatch.delenv(v, raising=False)
+    monkeypatch.setenv("FKC_CUS", "256")
+    assert _plan(1, N, K, D, 1, 0)[0] == (5 if kept else 3)
+
+
 def test_workspace_sizes():
     from flash_kmeans_cuda import _lib
     L = _lib.lib

@@ -225,6 +225,14 @@ def test_kept_scores_at_small_k(monkeypatch, dtype, B, N, K, D):
     assert not np.isin(got, [K - 1, 17]).any()
 
 
+@pytest.mark.parametrize("B,N,K,D", [
+    (1, 65537, 193, 128), (1, 65600, 257, 128), (1, 200001, 449, 128), (1, 196609, 385, 64),
+])
+def test_kept_scores_in_partial_stages(monkeypatch, B, N, K, D):
+    assert _plan(B, N, K, D, "f16")[0] == 5
+    test_kept_scores_at_small_k(monkeypatch, "f16", B, N, K, D)
+
+
 RESIDENT_CASES = [
     # (B, N, K, D): one centroid, K below and not a multiple of 16, ragged N,
     # batches, c4's shape at reduced N, and the largest tables that fit one

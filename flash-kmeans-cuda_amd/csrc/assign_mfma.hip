@@ -1651,17 +1651,15 @@ static Plan plan_filled(int64_t B, int64_t N, int64_t K, int64_t D,
   return p;
 }
 
-// Calls of fewer points keep the slice counts of plan_filled, by which their
-// callers' small workspaces have always been sized.
-constexpr int64_t kShortSliceMinPoints = 1000;
-
 // Modelled time (us, without the launch) of w workgroups per CU that score
 // kspan rows each: a lone wave's 16-row block takes its fragment reads (42
 // cycles per 32 features) and its MFMAs in turn, several share the matrix
 // pipe (19 cycles per tile and 32 features, stalls included) or the LDS (34);
 // a workgroup's start and end cost 2.5 us with kept scores and 3 + 0.7 per 32
 // features with the re-score; merging S slices 3 + 0.03 S.  Fitted to fp16
-// launches of 1000 .. 32768 points.
+// launches of 1000 .. 32768 points; fewer points launch the same grids as 1000
+// and follow it too ((1, 4096, 128) 32 -> 12 us, (64, 10000, 64) 29 -> 13,
+// (500, 4096, 128) 34 -> 13, (40, 65536, 64) 32 -> 17).
 static double grid_model(const Plan& p, int64_t wgs, int64_t cus) {
   const int64_t w = (wgs + cus - 1) / cus;
   const double cycles = std::max(42.0 + 16.0 * p.pt,
@@ -1684,9 +1682,7 @@ static Plan plan_assign(int64_t B, int64_t N, int64_t K, int64_t D,
                         bool can_slice) {
   const DeviceShape dev = device_shape();
   const Plan p = plan_filled(B, N, K, D, can_slice, dev);
-  if (!can_slice || p.exact || p.resident || K <= FKC_EXACT_MAX_K ||
-      B * N < kShortSliceMinPoints)
-    return p;
+  if (!can_slice || p.exact || p.resident || K <= FKC_EXACT_MAX_K) return p;
   const int64_t cus = dev.cus;
   const int64_t old_wgs = grid_wgs(p.pt, B, N) * p.S;
   const double old = p.ds2 > 4 ? wide_model(p.ds2, p.pt, false, old_wgs, p.kspan,

@@ -253,6 +253,16 @@ def test_slices_of_wide_rows(monkeypatch):
                 assert need(1, N, K, D, 1) <= (2 * half if S > 1 else 0), (N, K, D)
 
 
+@pytest.mark.parametrize("N", [1, 64, 500, 999, 1000])
+@pytest.mark.parametrize("K,D", [(3000, 128), (4096, 128), (10000, 64), (2048, 256)])
+def test_few_points_take_short_slices(monkeypatch, N, K, D):
+    for v in ("FKC_NTILES", "FKC_KSPLIT"):
+        monkeypatch.delenv(v, raising=False)
+    monkeypatch.setenv("FKC_CUS", "256")
+    assert _plan(1, N, K, D, 1, 1)[5] < 1024
+    assert _plan(1, N, K, D, 1, 0)[4] == 1
+
+
 @pytest.mark.parametrize("N,K,D,kept", [
     # D = 128: where the last 128-row stage is at most half used, the exact
     # index's 64-row stages were up to 23% faster ...

@@ -334,6 +334,16 @@ def test_underfilled_grids_slice_k(monkeypatch, dtype, B, N, K, D):
     assert not np.isin(got, [K - 1, K // 2]).any()
 
 
+@pytest.mark.parametrize("B,N,K,D", [
+    (1, 1, 4096, 128), (1, 64, 3000, 256), (2, 250, 10000, 64), (1, 999, 4100, 128),
+    (3, 13, 65536, 64), (1, 40, 20000, 512),
+])
+def test_few_points_slice_k(monkeypatch, B, N, K, D):
+    """As above with less than 1000 points, and more slices than the merge
+    loads at a time."""
+    test_underfilled_grids_slice_k(monkeypatch, "f16", B, N, K, D)
+
+
 def test_sliced_assign_workspace_errors(monkeypatch):
     """fkc_euclid_assign_ws rejects a short or misaligned workspace with
     FKC_ERR_WORKSPACE before launching anything, and needs none when the

@@ -251,6 +251,17 @@ LoopBuffers carve_loop(void* ws, int64_t B, int64_t N, int64_t K, int64_t D,
   if (total) *total = c.used;
   return L;
 }
+// Shift slots of a loop whose update fuses the finalize.  The rows that raise
+// one slot wait for one another (about 4 ns each), and the check reads and
+// clears every slot (about 10 ns each), so the two are balanced.
+int shift_slots(int64_t B, int64_t N, int64_t K, int64_t D) {
+  const int64_t rows = B * std::min(K, N);  // clusters that have points
+  int n = 1;
+  while (n < kShiftSlots && 2 * n * kShiftStride <= B * K * D &&
+         2 * (int64_t)n * n < rows)
+    n *= 2;
+  return n;
+}
 struct UpdateBuffers {
   int32_t* sorted = nullptr;
   int32_t* perm = nullptr;
@@ -652,10 +663,7 @@ int lloyd_run(const void* x, const void* init, void* centroids,
   // of the workspace are whole 256-byte blocks); otherwise one slot per
   // iteration (raised by launch_finalize).
   const bool fuses = update_fuses_finalize(D);
-  int nslots = 1;
-  while (nslots < kShiftSlots && 2 * nslots * kShiftStride <= B * K * D)
-    nslots *= 2;
-  if (!fuses) nslots = 1;
+  const int nslots = fuses ? shift_slots(B, N, K, D) : 1;
   if (check) {
     zf.z2 = fuses ? L.sums : L.shift;
     zf.n2 = fuses ? (int64_t)nslots * kShiftStride : max_iters;

@@ -1335,15 +1335,15 @@ static double wide_model(int ds2, int pt, bool exact, int64_t wgs, int64_t span,
   };
   // Up to D = 192, 224, 256, 288 and 512, for 1, 2, 4 tiles.
   static const Cost cost[5][3] = {
-      {{2.2, 2.96, 1.29, 200}, {3.0, 3.9, 1.76, 175}, {4.3, 5.9, 0, 195}},
-      {{2.04, 2.65, 0, 200}, {2.58, 3.5, 0, 190}, {3.9, 5.6, 0, 175}},
-      {{1.69, 2.18, 0, 170}, {2.25, 3.2, 0, 166}, {3.85, 5.46, 0, 172}},
-      {{1.98, 2.6, 0, 170}, {3.43, 3.93, 0, 170}, {}},
-      {{1.77, 3.54, 1.77, 170}, {2.63, 3.4, 0, 170}, {}}};
+      {{2.2, 2.96, 1.29, 230}, {3.0, 3.9, 1.76, 185}, {4.3, 5.9, 0, 193}},
+      {{2.04, 2.65, 0, 245}, {2.58, 3.5, 0, 190}, {3.9, 5.6, 0, 172}},
+      {{1.69, 2.18, 0, 222}, {2.25, 3.2, 0, 168}, {3.85, 5.46, 0, 170}},
+      {{1.98, 2.6, 0, 225}, {3.43, 3.93, 0, 145}, {}},
+      {{1.77, 3.54, 1.77, 350}, {2.63, 3.4, 0, 160}, {}}};
   const int w = ds2 <= 6 ? 0 : ds2 <= 9 ? ds2 - 6 : 4;
   Cost c = cost[w][pt == 1 ? 0 : pt == 2 ? 1 : 2];
   if (exact && ds2 == 9 && pt == 2) {
-    c = {3.24, 3.77, 1.56, 170};  // here three workgroups fit a CU
+    c = {3.24, 3.77, 1.56, 145};  // here three workgroups fit a CU
   } else if (exact) {
     c.one *= 1.2;
     c.two *= 1.06;

@@ -468,9 +468,9 @@ def test_whole_slices_are_enough(monkeypatch, B, N, K, D, nbytes):
 
 
 @pytest.mark.parametrize("B,N,K,D,dtype", [(1, 140000, 40, 24, "f32"), (1, 140000, 33, 37, "f16")])
-def test_vector_route_one_lane_per_point(B, N, K, D, dtype):
-    """The VALU route with one lane per point (grids of >= 512 workgroups:
-    N >= 131072) against the oracle, fp32 and an odd fp16 width."""
+def test_fp32_route_with_many_points(B, N, K, D, dtype):
+    """Grids of many waves per SIMD against the oracle, fp32 and an odd fp16
+    width."""
     x, c = _data(B, N, K, D, dtype, seed=N + D)
     got = _gpu_assign(x, c, dtype)
     _check(x, c, dtype, got, max_frac=1e-3)
@@ -494,40 +494,47 @@ def test_fp16_odd_widths_use_fp32_route(D):
 
 
 @pytest.mark.parametrize("B,N,K,D,dtype", [
-    (1, 4096, 64, 128, "f32"),    # c1: sixteen lanes per point
-    (2, 1000, 100, 36, "f32"),    # D not a multiple of the 32-feature chunk
+    (1, 4096, 64, 128, "f32"),    # the smallest benchmark shape
+    (2, 1000, 100, 36, "f32"),    # a partial last feature group
     (1, 513, 1, 16, "f32"),       # one centroid
     (3, 70, 10, 4, "f32"),        # fewer points than a workgroup holds
     (1, 3000, 60, 44, "f16"),     # odd-width 16-bit rows on the fp32 route
     (2, 777, 90, 52, "bf16"),
 ])
-def test_valu_resident_table_matches_tiled(monkeypatch, B, N, K, D, dtype):
-    """The vector route's table-resident kernel (table and points loaded
-    into LDS once, no barrier after) against the tiled kernel bit for bit,
-    with x_sq passed and computed in the kernel, and against the oracle."""
+def test_fp32_route_small_tables(B, N, K, D, dtype):
+    """Small tables, x_sq passed and computed in the kernel, against the
+    oracle.  (The plans are compared with one another in
+    test_fp32_plans_agree.)"""
     x, c = _data(B, N, K, D, dtype, seed=N * 3 + K + D)
-    monkeypatch.setenv("FKC_RESIDENT", "1")
-    got_r = _gpu_assign(x, c, dtype)
-    got_r2 = _gpu_assign(x, c, dtype, with_xsq=False)
-    monkeypatch.setenv("FKC_RESIDENT", "0")
-    got_t = _gpu_assign(x, c, dtype)
-    assert np.array_equal(got_r, got_t)
-    assert np.array_equal(got_r2, got_t)
-    _check(x, c, dtype, got_r, max_frac=1e-3 if B * N >= 4096 else None)
+    got = _gpu_assign(x, c, dtype)
+    assert np.array_equal(got, _gpu_assign(x, c, dtype, with_xsq=False))
+    _check(x, c, dtype, got, max_frac=1e-3 if B * N >= 4096 else None)
+
+
+def _fma(a, b, c):
+    """fp32 a * b + c rounded once: the product is exact in float64, the sum's
+    rounding error is known there, and a sum rounded to odd by it rounds to
+    fp32 as the exact one does."""
+    a, b, c = (np.asarray(v, np.float64) for v in (a, b, c))
+    p = a * b
+    s = np.asarray(p + c)
+    t = s - p
+    err = (p - (s - t)) + (c - t)
+    bits = s.view(np.int64)
+    odd = np.isfinite(s) & (err != 0) & (bits & 1 == 0)
+    bits[odd] += np.where((err > 0) == (s > 0), 1, -1)[odd]
+    return s.astype(np.float32)
 
 
 def _chain_labels(x, c, x_sq, c_sq):
     """Labels of the fp32 route restated on the CPU: dot products as one
-    fused multiply-add chain in feature order (each step exact in 80-bit
-    arithmetic, then rounded to fp32), the clamped distance, the first
+    fused multiply-add chain in feature order, the clamped distance, the first
     minimum below FLT_MAX.  x (n, D), c (K, D), all fp32 values."""
-    ld = np.longdouble
-    with np.errstate(invalid="ignore", over="ignore"):
+    with np.errstate(invalid="ignore", over="ignore", under="ignore"):
         acc = np.zeros((x.shape[0], c.shape[0]), np.float32)
         for d in range(x.shape[1]):
-            acc = (ld(acc) + ld(x[:, d, None]) * ld(c[None, :, d])).astype(np.float32)
-        t = x_sq[:, None] + c_sq[None, :]
-        dist = (ld(t) - 2 * ld(acc)).astype(np.float32)
+            acc = _fma(x[:, d, None], c[None, :, d], acc)
+        dist = _fma(np.float32(-2), acc, x_sq[:, None] + c_sq[None, :])
         dist = np.where(dist > 0, dist, np.float32(0))
     first = dist.argmin(1)
     return np.where(dist.min(1) < np.finfo(np.float32).max, first, 0)
@@ -552,8 +559,6 @@ FP32_CHAIN_CASES = [
 def test_fp32_route_is_the_fma_chain(B, N, K, D, dtype):
     """Bit for bit, ties, NaN and infinities among them, with x_sq passed and
     computed by the kernel (all points, or 300 of a large N)."""
-    from flash_kmeans_cuda import _C, synth
-    from flash_kmeans_cuda.ops import row_sqnorm
     rng = np.random.default_rng(N + K + D)
     xf = rng.standard_normal((B, N, D)).astype(np.float32)
     cf = rng.standard_normal((B, K, D)).astype(np.float32)
@@ -567,22 +572,45 @@ def test_fp32_route_is_the_fma_chain(B, N, K, D, dtype):
         xf[:, 13] *= 1e4
         cf[:, K // 2, D - 1] = -np.inf
         xf[:, 17] = cf[:, 0]
+    pick = np.arange(N) if N <= 5000 else np.r_[0:100, N - 100:N, rng.integers(0, N, 100)]
+    _check_chain(xf, cf, dtype, pick)
+
+
+def _check_chain(xf, cf, dtype, pick):
+    """GPU labels of the points `pick`, with x_sq passed and computed by the
+    kernel, against _chain_labels; returns those of the first batch row."""
+    from flash_kmeans_cuda import _C, synth
+    from flash_kmeans_cuda.ops import row_sqnorm
     xt, ct = synth.to_torch(O.from_f32(xf, dtype), dtype), synth.to_torch(O.from_f32(cf, dtype), dtype)
     xs, cs = row_sqnorm(xt), row_sqnorm(ct)
     got = _C.euclid_assign(xt, ct, xs, cs).cpu().numpy()
     own = _C.euclid_assign(xt, ct, torch.empty(0, device="cuda"), cs).cpu().numpy()
-    pick = np.arange(N) if N <= 5000 else np.r_[0:100, N - 100:N, rng.integers(0, N, 100)]
-    for b in range(B):
+    for b in range(len(xf)):
         xv, cv = xt[b].float().cpu().numpy()[pick], ct[b].float().cpu().numpy()
         csb = cs[b].cpu().numpy()
         ref = _chain_labels(xv, cv, xs[b].cpu().numpy()[pick], csb)
         assert np.array_equal(got[b, pick], ref)
-        with np.errstate(invalid="ignore", over="ignore"):
+        with np.errstate(invalid="ignore", over="ignore", under="ignore"):
             sq = np.zeros(len(pick), np.float32)
-            for d in range(D):
-                v = np.longdouble(xv[:, d])
-                sq = (np.longdouble(sq) + v * v).astype(np.float32)
+            for d in range(xf.shape[2]):
+                sq = _fma(xv[:, d], xv[:, d], sq)
         assert np.array_equal(own[b, pick], _chain_labels(xv, cv, sq, csb))
+    return got[0, pick]
+
+
+@pytest.mark.parametrize("scale", [1e-19, 3e-21, 1e-22, 4e17, 3e18])
+@pytest.mark.parametrize("B,N,K,D,dtype", [
+    (1, 1000, 64, 64, "f32"), (2, 500, 33, 37, "f32"), (1, 300, 70, 520, "f32"),
+    (1, 999, 40, 21, "bf16"), (1, 131073, 20, 12, "f32"),
+])
+def test_fp32_chain_at_the_ends_of_the_range(B, N, K, D, dtype, scale):
+    """Rows whose products and sums are subnormal, or overflow: still the
+    chain bit for bit, and more than one label."""
+    rng = np.random.default_rng(N + K)
+    xf = (rng.standard_normal((B, N, D)) * scale).astype(np.float32)
+    cf = (rng.standard_normal((B, K, D)) * scale).astype(np.float32)
+    labels = _check_chain(xf, cf, dtype, np.arange(min(N, 1000)))
+    assert scale == 3e18 or len(np.unique(labels)) > 1
 
 
 def _plan(B, N, K, D, dtype):

@@ -517,7 +517,7 @@ def main() -> int:
                                if args.config in REF_ASSIGN_TFLOPS else None),
         "ms_per_iter_ref_method": round(min(one), 5),
         "roofline": {
-            "bound": "valu" if f32 else "mfma",
+            "bound": "mfma",
             "achieved": round(assign_tflops, 2),
             "peak": peak,
             "unit": "TFLOP/s",

@@ -41,10 +41,10 @@ __device__ inline double wave_sum_f64(double v) {
 }
 
 // NI: 64-column slices of a row (D <= 64 NI), or 0 for any D, one row at a
-// time.  With NI known the rows are loaded in batches (64 elements of x and
-// 64 of the centroids in flight per lane) and accumulated in row order, the
-// same sums: one row at a time left the kernel waiting for a round trip per
-// row ((1, 262144, 4096, 128) fp16 62 us, and 40 us for 4096 sampled rows on
+// time.  With NI known the rows are loaded in batches (16, 32, 64 and 64
+// elements of x in flight per lane for NI = 1, 2, 4, 8, and as many of the
+// centroids) and accumulated in row order, the same sums: one row at a time
+// left the kernel waiting for a round trip per row ((1, 262144, 4096, 128) fp16 62 us, and 40 us for 4096 sampled rows on
 // 16 workgroups).  Bound by the loads: 2 D bytes of x per row from HBM and as
 // many of its centroid from the caches.
 template <int DT, int NI>

@@ -9,12 +9,13 @@
 // D % 8 != 0 or D > 512, and FKC_ASSIGN_FORCE_SAFE (api.cpp:12-25).
 //
 // v_mfma_f32_16x16x4_f32 and v_mfma_f32_32x32x2_f32 add their products to
-// the accumulator as a chain of fused multiply-adds in k order (a probe
-// compared 2.5 million results, subnormals, infinities and NaN among them,
-// with fmaf on the host: no bit differed), so a sequence of them over the
+// the accumulator as a chain of fused multiply-adds in k order (the tests of
+// this route compare its labels bit for bit with that chain, with subnormal,
+// overflowing, infinite and NaN rows among them), so a sequence of them over the
 // features gives the chain's bits at the matrix cores' fp32 rate (133 and 149
 // TFLOP/s measured in registers alone; 78 is the vector peak without packed
-// instructions).
+// instructions).  Norms that the caller leaves out are the same chain: the
+// points scored against themselves, read from the diagonal.
 //
 // Operands: A = M centroids x 64 / M features, B = as many features x M
 // points, so lane l holds centroid (A) or point (B) l % M.  Both are loaded

@@ -54,6 +54,9 @@ int launch_assign_mfma(const void* x, const void* c, const float* c_sq,
 namespace {
 
 constexpr int FT = 256;  // threads: four waves
+// assign_rows_kernel: widest rows, most centroids, floats per row in LDS.
+constexpr int kRowsMaxD = 32, kRowsMaxK = 8;
+__host__ __device__ constexpr int rows_ld(int D) { return 4 * (D / 4 | 1); }
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
@@ -566,7 +569,8 @@ __device__ inline void take_better(float& b, int& i, float ob, int oi) {
 // swaps, each group ending with one tile.  At (1, 3000000, 8, D) fp32, us, the
 // vector kernel (one lane per point), the kernel above, this one: D = 1 28 /
 // 44 / 24, D = 8 33 / 50 / 29, D = 16 40 / 41 / 39 (216 MB: 5.5 TB/s, partly
-// from the cache); D = 24 57 / 70 / 66.
+// from the cache); D = 24 57 / 70 / 66.  (Those of whole quads take
+// assign_rows_kernel since.)
 template <int DT, int G, int KT>
 __global__ void __launch_bounds__(FT, G == 1 ? 4 : 2)
 assign_few_kernel(const typename Elem<DT>::T* __restrict__ x,
@@ -709,6 +713,92 @@ assign_few_kernel(const typename Elem<DT>::T* __restrict__ x,
   }
 }
 
+// KM centroids at most, rows of whole quads and many points: one lane per
+// point.  A workgroup's rows pass through LDS so that they are loaded as one
+// contiguous block; every lane reads the same centroids from LDS.  Bound by
+// the loads: at (1, 3000000, 4, D) fp32, us, the vector kernel that passed
+// everything through LDS, assign_few_kernel, this one: D = 8 29 / 29 / 22,
+// D = 16 34 / 39 / 33, D = 24 52 / 65 / 53 (312 MB: 5.9 TB/s, partly from the
+// cache); norms left out cost it nothing.
+template <int DT, int KM>
+__global__ void __launch_bounds__(FT, 5)
+assign_rows_kernel(const typename Elem<DT>::T* __restrict__ x,
+                   const typename Elem<DT>::T* __restrict__ c,
+                   const float* __restrict__ x_sq,
+                   const float* __restrict__ c_sq, int32_t* __restrict__ ids,
+                   int N, int K, int D, const int32_t* __restrict__ ctrl) {
+  using T = typename Elem<DT>::T;
+  using Raw = typename Quad<DT>::Raw;
+  constexpr int QM = kRowsMaxD / 4;  // quads of a row, at most
+  if (loop_done(ctrl)) return;
+  // Rows of an odd number of quads: lanes that read their own rows spread
+  // over the banks.
+  extern __shared__ __attribute__((aligned(16))) float s_x[];
+  __shared__ __attribute__((aligned(16))) float s_c[KM][kRowsMaxD];
+  __shared__ float s_q[KM];
+  static_assert(KM * kRowsMaxD <= FT, "one centroid value per thread");
+  const int tid = threadIdx.x, b = blockIdx.y;
+  const int n0 = blockIdx.x * FT, n = n0 + tid;
+  const int qd = D / 4, nq = min(FT, N - n0) * qd, ld = rows_ld(D);
+  const T* xb = x + ((size_t)b * N + n0) * D;
+  const T* cb = c + (size_t)b * K * D;
+  float xs = 0.f;
+  Raw v[QM];
+#pragma unroll
+  for (int i = 0; i < QM; ++i)
+    if (i < qd)
+      v[i] = *reinterpret_cast<const Raw*>(xb + 4 * min(i * FT + tid, nq - 1));
+  if (x_sq != nullptr) xs = x_sq[(size_t)b * N + min(n, N - 1)];
+  if (tid < KM * kRowsMaxD) {
+    const int k = tid / kRowsMaxD, d = tid % kRowsMaxD;
+    s_c[k][d] = k < K && d < D ? Elem<DT>::load(cb[k * D + d]) : 0.f;
+  }
+  if (tid < KM) s_q[tid] = c_sq[(size_t)b * K + min(tid, K - 1)];
+  int r = tid / qd, q = tid - r * qd;
+  const int dr = FT / qd, dq = FT - dr * qd;
+#pragma unroll
+  for (int i = 0; i < QM; ++i)
+    if (i < qd) {
+      *reinterpret_cast<f32x4*>(s_x + r * ld + 4 * q) = Quad<DT>::cvt(v[i]);
+      r += dr;
+      q += dq;
+      if (q >= qd) {
+        q -= qd;
+        ++r;
+      }
+    }
+  __syncthreads();
+  const f32x4* row = reinterpret_cast<const f32x4*>(s_x + tid * ld);
+  float acc[KM], own = 0.f;
+#pragma unroll
+  for (int k = 0; k < KM; ++k) acc[k] = 0.f;
+  for (int i = 0; i < qd; ++i) {
+    const f32x4 xv = row[i];
+    if (x_sq == nullptr) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) own = fmaf(xv[e], xv[e], own);
+    }
+#pragma unroll
+    for (int k = 0; k < KM; ++k) {
+      const f32x4 cv = *reinterpret_cast<const f32x4*>(&s_c[k][4 * i]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[k] = fmaf(xv[e], cv[e], acc[k]);
+    }
+  }
+  if (x_sq == nullptr) xs = own;
+  float best = FLT_MAX;
+  int bidx = 0;
+#pragma unroll
+  for (int k = 0; k < KM; ++k)
+    if (k < K) {
+      const float dist = fmaf(-2.0f, acc[k], xs + s_q[k]);
+      const float nb = __builtin_amdgcn_fmed3f(dist, 0.f, best);
+      bidx = nb < best ? k : bidx;
+      best = nb;
+    }
+  if (n < N) ids[(size_t)b * N + n] = bidx;
+}
+
 // Bound by HBM at many rows.  R rows per wave, their loads in flight together:
 // one row per wave waits for a round trip with 2 to 8 bytes per lane
 // outstanding.  One and four rows, us: 65536 x 128 fp16 11.3 / 6.2, 100000 x
@@ -759,9 +849,9 @@ row_sqnorm_kernel(const typename Elem<DT>::T* __restrict__ src,
   }
 }
 
-// The launch of a shape: instruction shape m, m-point tiles per wave (pt),
-// 16-centroid tiles at a time (ct: rows above D = 512, and the few-centroid
-// kernel's KT), waves of a workgroup that share their points and split K (ks).
+// The launch of a shape: instruction shape m (64: one lane per point), m-point
+// tiles per wave (pt), 16-centroid tiles at a time (ct: rows above D = 512, and
+// the few-centroid kernel's KT; one lane per point: KM), waves of a workgroup that share their points and split K (ks).
 struct F32Plan {
   int m, pt, ct, ks;
 };
@@ -851,14 +941,27 @@ F32Plan plan_wide(int64_t B, int64_t N, int64_t K) {
   return best;
 }
 
-enum F32Kind { kChain, kWide, kFew };
+// Where assign_rows_kernel is taken, against the better of the two above, at
+// (1, N, K, D) fp32, us: N = 400000: (8, 24) 11 / 11, (4, 20) 10 / 7, (8, 32)
+// 15 / 14; N = 3000000: (8, 8) 29 / 23, (8, 16) 39 / 34, (8, 24) 65 / 55, (8, 32)
+// 82 / 76.
+bool f32_rows(int64_t B, int64_t N, int64_t K, int64_t D) {
+  return K <= kRowsMaxK && D <= kRowsMaxD && D % 4 == 0 && N >= 1024 &&
+         B * N >= 131072;
+}
+
+enum F32Kind { kChain, kWide, kFew, kRows = 8 };  // as in fkc_assign_plan
 
 F32Kind f32_kind(int64_t B, int64_t N, int64_t K, int64_t D) {
-  return D > 512 ? kWide : f32_few(B, N, K, D) ? kFew : kChain;
+  return D > 512                 ? kWide
+         : f32_rows(B, N, K, D) ? kRows
+         : f32_few(B, N, K, D)  ? kFew
+                                : kChain;
 }
 
 F32Plan f32_plan(F32Kind kind, int64_t B, int64_t N, int64_t K, int64_t D) {
   if (kind == kWide) return plan_wide(B, N, K);
+  if (kind == kRows) return {64, 1, K <= 4 ? 4 : 8, 1};
   if (kind == kFew) return {16, 4, D > 16 || K <= 16 ? 1 : K <= 32 ? 2 : 3, 1};
   return plan_f32(B, N, K, D);
 }
@@ -872,6 +975,17 @@ int launch_f32_t(const void* x, const void* c, const float* x_sq,
   const F32Plan p = f32_plan(kind, B, N, K, D);
   const int64_t per = p.m * p.pt * (4 / p.ks);  // points per workgroup
   dim3 grid((unsigned)((N + per - 1) / per), (unsigned)B);
+  if (kind == kRows) {
+    auto rows = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, grid, dim3(FT),
+                         (size_t)FT * rows_ld((int)D) * sizeof(float), s,
+                         static_cast<const T*>(x), static_cast<const T*>(c),
+                         x_sq, c_sq, ids, (int)N, (int)K, (int)D, ctrl);
+      return check_launch("assign_rows");
+    };
+    return p.ct == 4 ? rows(assign_rows_kernel<DT, 4>)
+                     : rows(assign_rows_kernel<DT, 8>);
+  }
   if (kind == kFew) {
     // One round of resident workgroups (4 per CU), or two of 6 for the
     // smallest: us at 3, 4, 6, 8, 12 per CU, (1, 3000000, 8, 8) 41 / 34 / 28 /

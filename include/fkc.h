@@ -336,10 +336,11 @@ FKC_CAPI size_t fkc_kmeans_sort_recounts_offset(int64_t B, int64_t N, int64_t K,
  * plan; slices: with a workspace of fkc_euclid_assign_fast_workspace_bytes.
  *   plan[0] kernel: 0 fp32 chains (D <= 512), 1 fp32 wide rows, 2 fp32 few
  *           centroids; 16-bit MFMA: 3 exact index, 4 re-score, 5 kept scores,
- *           6 whole table in one stage, 7 centroid-resident
- *   plan[1] edge of a score block (16 or 32)
+ *           6 whole table in one stage, 7 centroid-resident; 8 fp32 with one
+ *           lane per point
+ *   plan[1] edge of a score block (16 or 32; kernel 8: points of a wave)
  *   plan[2] point tiles per wave
- *   plan[3] centroid tiles at a time (kernels 1 and 2)
+ *   plan[3] centroid tiles at a time (kernels 1 and 2; kernel 8: centroids)
  *   plan[4] parts of K: waves of a workgroup (fp32), slices (16-bit)
  *   plan[5] centroid rows per slice
  */

@@ -658,9 +658,10 @@ def test_fp32_plans_agree(monkeypatch, B, N, K, D, dtype, cus):
     # three centroid tiles, 16 features filled and passed, several points
     # groups per wave and a ragged last one, batches
     (1, 131073, 1, 1, "f32"), (2, 70001, 5, 3, "f32"), (1, 140000, 16, 16, "f32"),
+    (1, 140000, 8, 9, "f32"), (1, 140000, 9, 8, "f32"),
     (1, 140000, 17, 8, "f32"), (1, 140000, 33, 13, "f32"), (1, 140000, 48, 12, "f32"),
     (1, 140000, 16, 24, "f32"), (4, 70000, 3, 17, "f32"), (1, 262145, 20, 5, "f16"),
-    (1, 140000, 47, 15, "bf16"), (3, 50000, 4, 20, "bf16"),
+    (1, 140000, 47, 15, "bf16"), (3, 50000, 4, 19, "bf16"),
 ])
 @pytest.mark.parametrize("cus", ["16", "256"])
 def test_few_centroids_of_few_features(monkeypatch, cus, B, N, K, D, dtype):
@@ -668,6 +669,20 @@ def test_few_centroids_of_few_features(monkeypatch, cus, B, N, K, D, dtype):
     chain, with one and with many groups of points per wave."""
     monkeypatch.setenv("FKC_CUS", cus)
     assert _plan(B, N, K, D, dtype)[0] == 2
+    test_fp32_route_is_the_fma_chain(B, N, K, D, dtype)
+
+
+@pytest.mark.parametrize("B,N,K,D,dtype", [
+    # one quad and eight, odd and even numbers of them, one centroid and all,
+    # a ragged last workgroup, batches, each type
+    (1, 131073, 1, 4, "f32"), (1, 140000, 8, 32, "f32"), (2, 70001, 3, 12, "f32"),
+    (1, 140000, 5, 16, "f32"), (3, 50000, 4, 28, "bf16"), (1, 262145, 8, 20, "f16"),
+    (128, 1030, 7, 8, "f32"),
+])
+def test_one_lane_per_point(B, N, K, D, dtype):
+    """Up to eight centroids of whole quads and many points, bit for bit the
+    chain."""
+    assert _plan(B, N, K, D, dtype)[0] == 8
     test_fp32_route_is_the_fma_chain(B, N, K, D, dtype)
 
 
@@ -704,7 +719,7 @@ def test_few_points_or_centroids_do_not_wait():
     """Shapes that once cost a round trip per feature or per group of
     features.  Ratios between calls, measured before and after: norms in the
     kernel 5.8 -> 1.6 and 5.3 -> 1.7; rows of 768 against 512 features 7.5 ->
-    1.2; rows of 8 against 16 features, many points, 1.3 -> 0.75."""
+    1.2; rows of 8 against 16 features, many points, 1.3 -> 0.65."""
     for shape in ((1, 35, 5, 768), (1, 1000, 4, 768)):
         assert _assign_us(*shape, given=False) < 3 * _assign_us(*shape)
     assert _assign_us(1, 1000, 4, 768) < 3 * _assign_us(1, 1000, 4, 512)

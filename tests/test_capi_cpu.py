@@ -218,6 +218,7 @@ def _plan(B, N, K, D, dtype, slices):
     # Shapes where more tiles per wave leave a last round of workgroups nearly
     # empty (two tiles, or one, were 10 to 20% faster than four, or two) ...
     (150000, 512, 160, 2), (150000, 2048, 192, 2), (200000, 64, 160, 2), (400000, 128, 136, 2),
+    (200000, 64, 256, 2),
     (150000, 300, 192, 2), (24000, 1000, 264, 1), (24000, 300, 264, 1), (80000, 1000, 264, 1),
     # ... and where they fill it.
     (262144, 512, 160, 4), (262144, 2048, 256, 4), (524288, 1000, 192, 4), (131072, 2048, 512, 2),
